@@ -58,6 +58,9 @@ SIGNATURES = {
                             _sz, _u32, _u32, _u32, _u32, _u32, _u32, _u32, _u32, _p],
     "aoakv_prefill_with_paged_kv_cache": [_p, _p, _p, _p, _u32, _u32, _u32, _u32, _u32,
                                           _u32, _u32, _u32, _u32, _p],
+    "aoakv_prefill_workspace_size": [_u32, _u32, _u32, _u32, _u32, _u32, _u32],
+    "aoakv_prefill_with_workspace": [_p, _p, _p, _p, _u32, _u32, _u32, _u32, _u32, _u32,
+                                     _u32, _u32, _u32, _p, _sz, _p],
     "aoakv_apply_rope_in_place": [_p, _p, _u32, _u32, _u32, _u32, _u32, _f32, _f32, _p],
     "aoakv_rms_norm_forward": [_p, _p, _p, _u32, _u32, _f32, _p],
     "aoakv_rope_append_kv_cache_decode": [_p, _p, _p, _u32, _u32, _p, _p, _p, _p, _p, _p, _p,
@@ -68,6 +71,7 @@ _RESTYPES = {
     "aoakv_version": ctypes.c_char_p,
     "aoakv_decode_workspace_size": _sz,
     "aoakv_layer_workspace_size": _sz,
+    "aoakv_prefill_workspace_size": _sz,
 }
 
 

@@ -389,7 +389,11 @@ def prefill_with_paged_kv_cache(q, kv_data, kv_indices, num_kv_pages: int, kv_la
         raise ValueError(f"q must be [L, Hq, {D}], got {tuple(q.shape)}")
     if o is None:
         o = torch.empty_like(q)
-    _lib.call("aoakv_prefill_with_paged_kv_cache", q.data_ptr(), o.data_ptr(), kv_data.data_ptr(),
+    n = _lib.load().aoakv_prefill_workspace_size(num_kv_pages, kv_last_page_len, q.shape[0],
+                                                 int(causal), q.shape[1], D, S)
+    # split keys: the chunks' partials, from torch's pool on this stream
+    ws = torch.empty(n, dtype=torch.uint8, device=q.device) if n else None
+    _lib.call("aoakv_prefill_with_workspace", q.data_ptr(), o.data_ptr(), kv_data.data_ptr(),
               kv_indices.data_ptr(), num_kv_pages, kv_last_page_len, q.shape[0], int(causal),
-              q.shape[1], H, D, S, layout, _stream())
+              q.shape[1], H, D, S, layout, _ptr(ws), n, _stream())
     return o

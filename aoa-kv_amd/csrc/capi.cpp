@@ -877,12 +877,33 @@ int aoakv_estimate_topk(const void* q, const void* metadata_data, const int32_t*
                               static_cast<hipStream_t>(stream));
 }
 
+size_t aoakv_prefill_workspace_size(uint32_t num_kv_pages, uint32_t kv_last_page_len,
+                                    uint32_t qo_len, uint32_t causal, uint32_t num_qo_heads,
+                                    uint32_t head_dim, uint32_t page_size) {
+  if (num_kv_pages == 0u || !aoakv::prefill_tuned_shape(head_dim, page_size)) return 0;
+  const uint64_t L = (uint64_t)(num_kv_pages - 1u) * page_size + kv_last_page_len;
+  if (qo_len == 0u || qo_len > L || L >= (1ull << 31)) return 0;
+  return aoakv::prefill_plan((uint32_t)L, qo_len, causal ? 1u : 0u, num_qo_heads, head_dim)
+      .workspace_bytes;
+}
+
 int aoakv_prefill_with_paged_kv_cache(const void* q, void* o, const void* kv_data,
                                       const int32_t* kv_indices, uint32_t num_kv_pages,
                                       uint32_t kv_last_page_len, uint32_t qo_len,
                                       uint32_t causal, uint32_t num_qo_heads,
                                       uint32_t num_kv_heads, uint32_t head_dim,
                                       uint32_t page_size, uint32_t layout, void* stream) {
+  return aoakv_prefill_with_workspace(q, o, kv_data, kv_indices, num_kv_pages, kv_last_page_len,
+                                      qo_len, causal, num_qo_heads, num_kv_heads, head_dim,
+                                      page_size, layout, nullptr, 0, stream);
+}
+
+int aoakv_prefill_with_workspace(const void* q, void* o, const void* kv_data,
+                                 const int32_t* kv_indices, uint32_t num_kv_pages,
+                                 uint32_t kv_last_page_len, uint32_t qo_len, uint32_t causal,
+                                 uint32_t num_qo_heads, uint32_t num_kv_heads,
+                                 uint32_t head_dim, uint32_t page_size, uint32_t layout,
+                                 void* workspace, size_t workspace_bytes, void* stream) {
   if (int e = check_shape(head_dim, page_size, layout, num_qo_heads)) return e;
   if (num_kv_heads == 0u || num_qo_heads % num_kv_heads != 0u)
     return fail(AOAKV_ERR_INVALID,
@@ -912,7 +933,8 @@ int aoakv_prefill_with_paged_kv_cache(const void* q, void* o, const void* kv_dat
   a.g = aoakv::make_geom(layout, num_kv_heads, page_size, head_dim);
   hipStream_t s = static_cast<hipStream_t>(stream);
   return hip_status(aoakv::prefill_tuned_shape(head_dim, page_size)
-                        ? aoakv::launch_prefill(a, page_size, head_dim, s)
+                        ? aoakv::launch_prefill(a, page_size, head_dim, workspace,
+                                                workspace_bytes, s)
                         : aoakv::launch_gen_prefill(a, head_dim, s),
                     "prefill_with_paged_kv_cache");
 }

@@ -184,7 +184,21 @@ struct PrefillArgs {
   uint32_t Hq;                // query heads, a multiple of H
   float sm_scale;
   PageGeom g;
+  // key tiles split into chunks (chunk_rcp != 0, see prefill_plan): items per
+  // query head and their partials
+  uint32_t chunk_rcp;
+  uint32_t per_head;
+  float* partial;
 };
+
+// How a prefill call's key tiles are split into chunks (chunk_rcp == 0: not),
+// and the workspace the chunks' partials take.
+struct PrefillPlan {
+  uint32_t chunk_rcp;
+  uint32_t per_head;
+  size_t workspace_bytes;
+};
+PrefillPlan prefill_plan(uint32_t L, uint32_t Lq, uint32_t causal, uint32_t Hq, uint32_t head_dim);
 
 // One decode layer in one launch (see layer_kernel in decode.hip).
 struct LayerArgs {
@@ -214,8 +228,9 @@ uint64_t layer_max_workgroups();  // one-launch layer grid limit (32-bit work-it
 hipError_t launch_decode(const DecodeArgs& a, uint32_t batch, hipStream_t s,
                          const EstimateArgs* self = nullptr);
 hipError_t launch_fill_u32(uint32_t* p, size_t n, uint32_t v, hipStream_t s);
+// workspace (may be null): split as prefill_plan says if it is large enough
 hipError_t launch_prefill(const PrefillArgs& a, uint32_t page_size, uint32_t head_dim,
-                          hipStream_t s);
+                          void* workspace, size_t workspace_bytes, hipStream_t s);
 
 // RMSNorm of `rows` fp16 rows of n elements (n a multiple of 8), one weight row.
 struct RmsNormArgs {

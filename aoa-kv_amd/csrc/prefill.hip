@@ -110,6 +110,29 @@ struct PfShape {
 template <int D>
 constexpr int pf_blocks_per_cu() { return D == 256 ? 1 : 2; }
 
+// Running max before a query's first visible key: below every score, and
+// finite, so a tile (or a whole chunk) with no visible key leaves
+// probabilities of 2^-inf = 0 and no inf - inf.
+constexpr float kPfNoMax = -1e30f;
+
+// Key tiles of query tile qt, and the chunks they are split into.
+__host__ __device__ inline uint32_t pf_tiles(uint32_t L, uint32_t Lq, uint32_t causal,
+                                             uint32_t qt) {
+  uint32_t qend = (qt + 1u) * kPfQueriesPerBlock;
+  qend = qend < Lq ? qend : Lq;
+  const uint32_t kend = causal ? L - Lq + qend : L;
+  return (kend + kPfTileKeys - 1) / kPfTileKeys;
+}
+// ceil(n / chunk) for n <= 2^25 tiles: chunk_rcp = floor(2^32 / chunk) + 1
+// rounds n - 1 tiles down exactly while n * chunk < 2^32.
+__host__ __device__ inline uint32_t pf_chunks(uint32_t n, uint32_t chunk_rcp) {
+  return (uint32_t)(((uint64_t)(n - 1u) * chunk_rcp) >> 32) + 1u;
+}
+// floats of one item's partial: O [D / 4][128 queries][4], m [128], l [128]
+__host__ __device__ constexpr size_t pf_partial_floats(int D) {
+  return (size_t)kPfQueriesPerBlock * (D + 2);
+}
+
 // S: tokens per page (1, 2, 4, 8, 16 or 32); D: head dim (64, 128 or 256).
 template <int S, int D>
 __global__ __launch_bounds__(kPfThreads, pf_blocks_per_cu<D>()) void prefill_kernel(PrefillArgs a) {
@@ -130,31 +153,44 @@ __global__ __launch_bounds__(kPfThreads, pf_blocks_per_cu<D>()) void prefill_ker
   const uint32_t L = a.L, Lq = a.Lq;
   const uint32_t nqt = (Lq + kPfQueriesPerBlock - 1) / kPfQueriesPerBlock;
   // XCD-aware work order.  Workgroup b runs on XCD b % 8, and each XCD has
-  // its own L2, so XCD x takes the contiguous range [x * per, (x+1) * per)
-  // of the head-major item list: all query tiles of a head (and of the
-  // query heads that share its kv head) run on one XCD, whose L2 then holds
-  // that head's K/V for all of them.  Within a head, heaviest tiles first.
-  const uint32_t per = (nqt * a.Hq + kXcds - 1) / kXcds;
-  const uint32_t item = (blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
-  if (item >= nqt * a.Hq) return;  // block-uniform: the last XCD's range is short
-  const uint32_t h = item / nqt;           // query head
+  // its own L2.  Items go heaviest query tile first over all heads, head
+  // fastest, so with a multiple of 8 heads XCD x has the heads of x alone:
+  // its Hq / 8 consecutive ones (sharing kv heads with GQA), whose K/V its L2
+  // then holds for the query tiles in flight.  The lightest tiles of every
+  // head come last and fill the CUs' ends.
+  const uint32_t per_head = a.chunk_rcp != 0u ? a.per_head : nqt;  // items
+  const uint32_t hs = blockIdx.x % a.Hq;
+  const uint32_t h = a.Hq % kXcds == 0u ? hs % kXcds * (a.Hq / kXcds) + hs / kXcds : hs;
   const uint32_t hkv = h / (a.Hq / a.H);   // its kv head (GQA groups share K/V)
-  const uint32_t qt = nqt - 1u - item % nqt;  // heaviest query tiles first
+  uint32_t qt = nqt - 1u, rank = blockIdx.x / a.Hq;
+  const uint32_t item = h * per_head + rank;  // its partial's place
+  uint32_t ntiles = 0u, nchunks = 1u;
+  if (a.chunk_rcp != 0u) {
+    for (;; --qt) {
+      ntiles = pf_tiles(L, Lq, a.causal, qt);
+      nchunks = pf_chunks(ntiles, a.chunk_rcp);
+      if (rank < nchunks || qt == 0u) break;
+      rank -= nchunks;
+    }
+  } else {
+    qt -= rank;
+    rank = 0u;
+    ntiles = pf_tiles(L, Lq, a.causal, qt);
+  }
+  // this item's key tiles
+  const uint32_t t0 = rank * ntiles / nchunks, t1 = (rank + 1u) * ntiles / nchunks;
   const uint32_t off = L - Lq;                 // position of query 0
   const uint32_t npages = (L + S - 1) / S;
 
   const uint32_t q = qt * kPfQueriesPerBlock + wave * kPfQueriesPerWave + c;
   const bool q_live = q < Lq;
   const uint32_t qpos = q_live ? off + q : L - 1u;  // last key this query sees
-  // keys this block needs: up to the last live query's position
-  uint32_t qlast = qt * kPfQueriesPerBlock + kPfQueriesPerBlock - 1u;
-  if (qlast >= Lq) qlast = Lq - 1u;
-  const uint32_t kend = a.causal ? off + qlast + 1u : L;
-  const uint32_t ntiles = (kend + kPfTileKeys - 1) / kPfTileKeys;
-  // keys this wave needs (waves above the diagonal skip tiles)
-  uint32_t wq_last = qt * kPfQueriesPerBlock + wave * kPfQueriesPerWave + kPfQueriesPerWave - 1u;
+  // keys this wave needs (waves above the diagonal skip tiles; a wave with no
+  // live query skips them all)
+  const uint32_t wq_first = qt * kPfQueriesPerBlock + wave * kPfQueriesPerWave;
+  uint32_t wq_last = wq_first + kPfQueriesPerWave - 1u;
   if (wq_last >= Lq) wq_last = Lq - 1u;
-  const uint32_t wave_kend = a.causal ? off + wq_last + 1u : L;
+  const uint32_t wave_kend = wq_first >= Lq ? 0u : a.causal ? off + wq_last + 1u : L;
 
   // ---- this lane's query, dims 16*s + 8*g .. +8 for s < D / 16
   half8 qreg[Sh::kKS];
@@ -243,7 +279,7 @@ __global__ __launch_bounds__(kPfThreads, pf_blocks_per_cu<D>()) void prefill_ker
   floatx16 acc_o[Sh::kDB];
 #pragma unroll
   for (int t = 0; t < Sh::kDB; ++t) acc_o[t] = floatx16{};
-  float m_run = -INFINITY, l_run = 0.f;  // running max of the unscaled scores
+  float m_run = kPfNoMax, l_run = 0.f;  // running max of the unscaled scores
   const float scale = a.sm_scale * kLog2e;
   // smallest query position of this wave: tiles with every key at or below
   // it (and below L) need no mask
@@ -330,7 +366,7 @@ __global__ __launch_bounds__(kPfThreads, pf_blocks_per_cu<D>()) void prefill_ker
     mt = pair_max(mt);
     // Lazy rescaling: the reference max m_run moves only when some query's
     // tile max exceeds it by more than 2^8 in probability (the first tile
-    // always moves it: every query sees key 0 there).  Otherwise
+    // with a visible key always moves it).  Otherwise
     // probabilities stay <= 256, exact in fp16 relative terms, and the
     // final o = O / l divides both by the same reference.
     const bool move = __builtin_amdgcn_ballot_w64((mt - m_run) * scale > 8.f) != 0;
@@ -350,7 +386,7 @@ __global__ __launch_bounds__(kPfThreads, pf_blocks_per_cu<D>()) void prefill_ker
     }
     lt = pair_sum(lt);
     if (move) {  // the reference moved for some query: rescale
-      const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * scale);  // m_run = -inf: 0
+      const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * scale);  // m_run = kPfNoMax: 0
       l_run = l_run * alpha;
 #pragma unroll
       for (int t = 0; t < Sh::kDB; ++t)
@@ -392,19 +428,19 @@ __global__ __launch_bounds__(kPfThreads, pf_blocks_per_cu<D>()) void prefill_ker
     }
   };
 
-  load_tile(s_buf0, page_of(0u));
-  PageIds phys_next = page_of(1u);
+  load_tile(s_buf0, page_of(t0));
+  PageIds phys_next = page_of(t0 + 1u);
   // two tiles per trip: even tiles in buffer 0, odd tiles in buffer 1
-  for (uint32_t it = 0; it < ntiles; it += 2) {
+  for (uint32_t it = t0; it < t1; it += 2) {
 #pragma unroll
     for (uint32_t u = 0; u < 2; ++u) {
       const uint32_t ti = it + u;
-      if (ti >= ntiles) break;  // uniform
+      if (ti >= t1) break;  // uniform
       // tile ti has landed in LDS (this wave's loads: vmcnt; the others':
       // the barrier), and every wave is done with the other buffer
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
-      if (ti + 1 < ntiles) {  // in flight during this tile's MFMAs
+      if (ti + 1 < t1) {  // in flight during this tile's MFMAs
         load_tile(u == 0u ? s_buf1 : s_buf0, phys_next);
         phys_next = page_of(ti + 2u);
       }
@@ -425,6 +461,25 @@ __global__ __launch_bounds__(kPfThreads, pf_blocks_per_cu<D>()) void prefill_ker
     }
   }
 
+  if (nchunks > 1u) {  // ---- a chunk's partial, for prefill_merge_kernel
+    float* part = a.partial + (size_t)item * pf_partial_floats(D);
+    float4* po = reinterpret_cast<float4*>(part) + wave * kPfQueriesPerWave + c;
+#pragma unroll
+    for (int j = 0; j < Sh::kDB * 4; ++j) {
+      const floatx16& x = acc_o[j / 4];
+      const int i0 = 4 * (j % 4);
+      // dims 32 (j / 4) + crow(i0, g) .. + 3
+      po[(8 * (j / 4) + 2 * (j % 4) + g) * kPfQueriesPerBlock] =
+          float4{x[i0], x[i0 + 1], x[i0 + 2], x[i0 + 3]};
+    }
+    if (g == 0) {
+      float* pm = part + kPfQueriesPerBlock * D + wave * kPfQueriesPerWave + c;
+      pm[0] = m_run;
+      pm[kPfQueriesPerBlock] = l_run;
+    }
+    return;
+  }
+
   // ---- o = O / l: lane holds its query's dims t*32 + crow(i, g)
   if (!q_live) return;
   const float inv_l = 1.f / l_run;
@@ -441,35 +496,142 @@ __global__ __launch_bounds__(kPfThreads, pf_blocks_per_cu<D>()) void prefill_ker
   }
 }
 
-hipError_t launch_prefill(const PrefillArgs& a, uint32_t page_size, uint32_t head_dim,
-                          hipStream_t s) {
+// Joins the chunks' partials of split query tiles: one workgroup per (query
+// head, query tile, 32 queries); thread t takes query t % 32 and D / 8 dims.
+template <int D>
+__global__ __launch_bounds__(kPfThreads) void prefill_merge_kernel(PrefillArgs a) {
   const uint32_t nqt = (a.Lq + kPfQueriesPerBlock - 1) / kPfQueriesPerBlock;
-  const uint32_t per = (nqt * a.Hq + kXcds - 1) / kXcds;
-  const dim3 grid(per * kXcds), block(kPfThreads);
-#define AOAKV_PF(S_, D_)                                                     \
-  if (page_size == S_ && head_dim == D_) {                                   \
-    hipLaunchKernelGGL((prefill_kernel<S_, D_>), grid, block, 0, s, a);      \
-    return hipGetLastError();                                                \
+  const uint32_t sub = blockIdx.x % 4u, x = blockIdx.x / 4u;
+  const uint32_t h = x / nqt, qt = x % nqt;
+  const uint32_t nchunks = pf_chunks(pf_tiles(a.L, a.Lq, a.causal, qt), a.chunk_rcp);
+  const uint32_t row = sub * 32u + threadIdx.x % 32u, j0 = threadIdx.x / 32u;
+  const uint32_t q = qt * kPfQueriesPerBlock + row;
+  if (nchunks == 1u || q >= a.Lq) return;
+  uint32_t item = h * a.per_head;  // the tile's first
+  for (uint32_t y = nqt - 1u; y > qt; --y)
+    item += pf_chunks(pf_tiles(a.L, a.Lq, a.causal, y), a.chunk_rcp);
+  const float scale = a.sm_scale * kLog2e;
+  const float* part = a.partial + (size_t)item * pf_partial_floats(D);
+  float m = kPfNoMax, l = 0.f;
+  for (uint32_t s = 0; s < nchunks; ++s)
+    m = fmaxf(m, part[s * pf_partial_floats(D) + kPfQueriesPerBlock * D + row]);
+  constexpr int kV = D / 32;  // 4-dim vectors per thread
+  float4 acc[kV] = {};
+  for (uint32_t s = 0; s < nchunks; ++s) {
+    const float* p = part + s * pf_partial_floats(D);
+    const float* pm = p + kPfQueriesPerBlock * D + row;
+    const float w = __builtin_amdgcn_exp2f((pm[0] - m) * scale);
+    l += pm[kPfQueriesPerBlock] * w;
+#pragma unroll
+    for (int v = 0; v < kV; ++v) {
+      const float4 y = reinterpret_cast<const float4*>(p)[(kV * j0 + v) * kPfQueriesPerBlock + row];
+      acc[v].x += y.x * w;
+      acc[v].y += y.y * w;
+      acc[v].z += y.z * w;
+      acc[v].w += y.w * w;
+    }
   }
-  AOAKV_PF(1, 128)
-  AOAKV_PF(2, 128)
-  AOAKV_PF(4, 128)
-  AOAKV_PF(8, 128)
-  AOAKV_PF(16, 128)
-  AOAKV_PF(32, 128)
-  AOAKV_PF(1, 64)
-  AOAKV_PF(2, 64)
-  AOAKV_PF(4, 64)
-  AOAKV_PF(8, 64)
-  AOAKV_PF(16, 64)
-  AOAKV_PF(32, 64)
-  AOAKV_PF(1, 256)
-  AOAKV_PF(2, 256)
-  AOAKV_PF(4, 256)
-  AOAKV_PF(8, 256)
-  AOAKV_PF(16, 256)
-  AOAKV_PF(32, 256)
-#undef AOAKV_PF
+  const float inv_l = 1.f / l;
+  f16* orow = a.o + ((size_t)q * a.Hq + h) * D + 4 * kV * j0;
+#pragma unroll
+  for (int v = 0; v < kV; ++v)
+    *reinterpret_cast<half4*>(orow + 4 * v) =
+        half4{(f16)(acc[v].x * inv_l), (f16)(acc[v].y * inv_l), (f16)(acc[v].z * inv_l),
+              (f16)(acc[v].w * inv_l)};
+}
+
+// The calls that are split, and into chunks of how many key tiles.  One item
+// (128 queries of a head) walks its key tiles one after the other, so few
+// items over a long context leave most CUs idle: 500 queries x 32 heads over
+// 16384 keys are 128 items of 256 tiles, 334 us (396 TFLOP/s); as 512 items
+// of 64 tiles, 151 us (878).  100 queries over 8192 keys: 165 -> 39 us; 300
+// over 16000 at 16 heads of dim 256: 641 -> 155.  A split costs its partials
+// (fp32, written and read once) and a second launch, so a call whose items
+// fill the chip is faster whole (3001 x 3001, 32 heads: 90 us, in chunks of
+// 32 tiles 110; 8192 x 8192: 585, in chunks of 64 659).  Measured step times decide: a CU
+// with k items resident takes t[k] us per tile of each (d64 0.92, 1.25, 1.8;
+// d128 1.3, 2.05; d256 2.56), the partials move at 4 TB/s, the joining launch
+// takes 5 us.  Against measured calls of 16 to 1536 items the estimate is
+// within 15%, and picks the best split or one within 10% of it.
+PrefillPlan prefill_plan(uint32_t L, uint32_t Lq, uint32_t causal, uint32_t Hq,
+                         uint32_t head_dim) {
+  constexpr uint32_t kCus = 256u;
+  constexpr float kStep[3][3] = {{0.92f, 1.25f, 1.8f}, {1.3f, 2.05f, 2.05f}, {2.56f, 2.56f, 2.56f}};
+  const float* step = kStep[head_dim == 64u ? 0 : head_dim == 128u ? 1 : 2];
+  const uint32_t occ = head_dim == 64u ? 3u : head_dim == 128u ? 2u : 1u;  // items per CU
+  const uint32_t slots = kCus * occ;
+  PrefillPlan best{};
+  const uint32_t nqt = (Lq + kPfQueriesPerBlock - 1) / kPfQueriesPerBlock;
+  const uint32_t nmax = pf_tiles(L, Lq, causal, nqt - 1u);
+  if ((uint64_t)nqt * Hq >= 2u * slots || nmax < 8u || nmax > 65535u) return best;
+  float best_us = 0.f;
+  // chunks of 2 / s of the longest item's tiles
+  for (uint32_t s : {2u, 3u, 4u, 6u, 8u, 10u, 12u, 16u, 20u, 24u, 32u, 40u, 48u, 64u, 96u, 128u}) {
+    const uint32_t chunk = (2u * nmax + s - 1u) / s;
+    if (chunk < 4u) break;
+    const uint32_t rcp = (uint32_t)((1ull << 32) / chunk) + 1u;
+    uint64_t items = 0u, partials = 0u, tiles = 0u;
+    for (uint32_t qt = 0; qt < nqt; ++qt) {
+      const uint32_t t = pf_tiles(L, Lq, causal, qt), c = pf_chunks(t, rcp);
+      items += c;
+      tiles += t;
+      partials += c > 1u ? c : 0u;
+    }
+    const uint32_t per_head = (uint32_t)items;
+    items *= Hq;
+    if (s > 2u && items > 4u * slots) break;
+    // all resident at once: the longest; else the CUs' rate, and half of the
+    // longest at the end
+    float us = items <= slots
+                   ? (float)chunk * step[(items + kCus - 1u) / kCus - 1u]
+                   : (float)(tiles * Hq) * step[occ - 1u] / (float)slots + 0.5f * chunk * step[0];
+    if (s > 2u)
+      us += 5.f + (float)(partials * Hq * pf_partial_floats((int)head_dim)) * 8.f / 4e6f;
+    if (s == 2u) {
+      best_us = 0.95f * us;  // a split has to be worth its launch
+    } else if (us < best_us) {
+      best_us = us;
+      best.chunk_rcp = rcp;
+      best.per_head = per_head;
+      best.workspace_bytes = items * pf_partial_floats((int)head_dim) * sizeof(float);
+    }
+  }
+  return best;
+}
+
+template <int D>
+static hipError_t launch_pf(const PrefillArgs& a, uint32_t page_size, hipStream_t s) {
+  const uint32_t nqt = (a.Lq + kPfQueriesPerBlock - 1) / kPfQueriesPerBlock;
+  const uint32_t items = (a.chunk_rcp != 0u ? a.per_head : nqt) * a.Hq;
+  const dim3 grid(items), block(kPfThreads);
+  switch (page_size) {
+    case 1: hipLaunchKernelGGL((prefill_kernel<1, D>), grid, block, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((prefill_kernel<2, D>), grid, block, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((prefill_kernel<4, D>), grid, block, 0, s, a); break;
+    case 8: hipLaunchKernelGGL((prefill_kernel<8, D>), grid, block, 0, s, a); break;
+    case 16: hipLaunchKernelGGL((prefill_kernel<16, D>), grid, block, 0, s, a); break;
+    case 32: hipLaunchKernelGGL((prefill_kernel<32, D>), grid, block, 0, s, a); break;
+    default: return hipErrorInvalidValue;
+  }
+  if (hipError_t e = hipGetLastError(); e != hipSuccess || a.chunk_rcp == 0u) return e;
+  hipLaunchKernelGGL(prefill_merge_kernel<D>, dim3(a.Hq * nqt * 4u), block, 0, s, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_prefill(const PrefillArgs& args, uint32_t page_size, uint32_t head_dim,
+                          void* workspace, size_t workspace_bytes, hipStream_t s) {
+  PrefillArgs a = args;
+  const PrefillPlan p = prefill_plan(a.L, a.Lq, a.causal, a.Hq, head_dim);
+  if (p.chunk_rcp != 0u && workspace != nullptr && workspace_bytes >= p.workspace_bytes) {
+    a.chunk_rcp = p.chunk_rcp;
+    a.per_head = p.per_head;
+    a.partial = static_cast<float*>(workspace);
+  }
+  switch (head_dim) {
+    case 64: return launch_pf<64>(a, page_size, s);
+    case 128: return launch_pf<128>(a, page_size, s);
+    case 256: return launch_pf<256>(a, page_size, s);
+  }
   return hipErrorInvalidValue;
 }
 

@@ -428,6 +428,25 @@ int aoakv_prefill_with_paged_kv_cache(const void* q, void* o, const void* kv_dat
                                       uint32_t num_kv_heads, uint32_t head_dim,
                                       uint32_t page_size, uint32_t layout, void* stream);
 
+/*
+ * aoakv_prefill_with_paged_kv_cache with a workspace: where the query tiles
+ * alone would leave the chip idle (few queries over a long context), their
+ * keys are split into chunks whose partial results (fp32) are joined by a
+ * second launch.  aoakv_prefill_workspace_size gives the bytes such a call
+ * takes (0: the call is not split).  workspace NULL or smaller: not split.
+ * The workspace needs no initialisation, is free again when the call's work
+ * on `stream` is done, and must be aligned to 16 bytes.
+ */
+size_t aoakv_prefill_workspace_size(uint32_t num_kv_pages, uint32_t kv_last_page_len,
+                                    uint32_t qo_len, uint32_t causal, uint32_t num_qo_heads,
+                                    uint32_t head_dim, uint32_t page_size);
+int aoakv_prefill_with_workspace(const void* q, void* o, const void* kv_data,
+                                 const int32_t* kv_indices, uint32_t num_kv_pages,
+                                 uint32_t kv_last_page_len, uint32_t qo_len, uint32_t causal,
+                                 uint32_t num_qo_heads, uint32_t num_kv_heads,
+                                 uint32_t head_dim, uint32_t page_size, uint32_t layout,
+                                 void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

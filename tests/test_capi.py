@@ -188,3 +188,23 @@ def test_noalloc_entry_point_rejects_without_gpu():
     # the error-word reader needs somewhere to put the bits
     rc = lib.aoakv_noalloc_error(None, 1, None)
     assert rc == _lib.AOAKV_ERR_INVALID and b"error_bits" in lib.aoakv_last_error()
+
+
+def test_prefill_workspace_is_for_few_queries_over_many_keys():
+    """Calls whose query tiles fill the chip take no workspace; a split one's
+    stays bounded (4 x 768 partials of 128 rows x 66 floats, 4 x 512 of 130 or
+    4 x 256 of 258)."""
+    from aoakv import _lib
+    size = _lib.load().aoakv_prefill_workspace_size
+    assert size(512, 16, 8192, 1, 32, 128, 16) == 0       # a long prompt
+    assert size(21, 13, 333, 1, 32, 128, 16) == 0         # a short one
+    assert size(1024, 16, 500, 1, 32, 128, 16) > 0        # a chunk after 16k tokens
+    assert size(1024, 16, 500, 1, 32, 128, 7) == 0        # not a shape of the split kernel
+    assert size(0, 1, 1, 1, 32, 128, 16) == 0 and size(1, 16, 17, 1, 32, 128, 16) == 0
+    for D, slots in ((64, 768), (128, 512), (256, 256)):
+        for pages in (64, 777, 4096, 65536):
+            for qo in (1, 100, 129, 1000, 4000):
+                for H in (1, 3, 8, 32, 256):
+                    n = size(pages, 5, min(qo, 16 * pages - 11), 1, H, D, 16)
+                    assert n % (4 * 128 * (D + 2)) == 0
+                    assert n <= 4 * slots * 4 * 128 * (D + 2)

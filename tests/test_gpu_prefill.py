@@ -186,3 +186,53 @@ def test_prefill_ignores_unwritten_slots_past_the_sequence(L):
     rows = np.unique(np.linspace(0, L - 1, 24).astype(np.int64))
     ref = sim.causal_prefill_rows(q, k, v, rows)
     assert np.abs(o[rows].astype(np.float32) - ref).max() <= 2e-3
+
+
+# (L, Lq, Hq, Hkv, D, page size, layout, causal): one ragged query tile, one
+# full and one of a single row, many heads that do not divide by 8, a page
+# per key, chunks of unequal length, unmasked queries
+SPLIT = [(2048, 64, 32, 32, 128, 16, HND, True), (1500, 129, 4, 2, 128, 16, NHD, True),
+         (2049, 128, 3, 3, 128, 1, HND, True), (1111, 17, 12, 3, 64, 8, NHD, True),
+         (1031, 5, 2, 1, 256, 32, HND, True), (3000, 300, 2, 2, 64, 16, HND, True),
+         (1200, 40, 4, 4, 128, 16, HND, False), (4099, 1, 8, 8, 128, 16, NHD, True)]
+
+
+@pytest.mark.parametrize("L,Lq,Hq,Hkv,D,S,layout,causal", SPLIT)
+def test_prefill_split_keys(L, Lq, Hq, Hkv, D, S, layout, causal):
+    """Few queries over a long context: the keys of a query tile are split into
+    chunks joined by a second launch (the call takes a workspace).  Held to
+    the fp64 oracle and, within the same bar, to the call without a workspace,
+    which is not split; the cache's unwritten slots are NaN."""
+    from aoakv import _lib, ops
+    from aoakv.utils import InferenceController, append_kv
+    _say(f"[prefill split] L={L} Lq={Lq} heads={Hq}/{Hkv} D={D} S={S} causal={causal}")
+    q = randn16(60 + L, (Lq, Hq, D), 0.5)
+    k = randn16(61 + L, (L, Hkv, D), 0.5)
+    v = randn16(62 + L, (L, Hkv, D), 0.5)
+    c = InferenceController(1, Hq, D, S, 64, L + S, torch.float16, DEV, layout=layout,
+                            num_kv_heads=Hkv, shuffle_seed=7)
+    c.kv_cache.buf_layer(0).fill_(float("nan"))
+    c.prepare_metadata(L)
+    c.begin_forward(L)
+    append_kv(torch.from_numpy(k).to(DEV), torch.from_numpy(v).to(DEV), c, 0)
+    qd, P, last = torch.from_numpy(q).to(DEV), len(c.kv_cache.indicies), c.kv_cache.last_page_len
+    assert _lib.load().aoakv_prefill_workspace_size(P, last, Lq, int(causal), Hq, D, S) > 0
+    o = ops.prefill_with_paged_kv_cache(qd, c.kv_cache.buf_layer(0), c.kv_indices_with_last, P,
+                                        last, layout, causal=causal)
+    whole = torch.empty_like(o)
+    _lib.call("aoakv_prefill_with_paged_kv_cache", qd.data_ptr(), whole.data_ptr(),
+              c.kv_cache.buf_layer(0).data_ptr(), c.kv_indices_with_last.data_ptr(), P, last, Lq,
+              int(causal), Hq, Hkv, D, S, layout, torch.cuda.current_stream().cuda_stream)
+    rows = np.unique(np.linspace(0, Lq - 1, 24).astype(np.int64))
+    kr, vr = np.repeat(k, Hq // Hkv, axis=1), np.repeat(v, Hq // Hkv, axis=1)
+    if causal:
+        ref = sim.causal_prefill_rows(q, kr, vr, rows)
+    else:
+        x = np.einsum("rhd,lhd->rhl", q[rows].astype(np.float64), kr.astype(np.float64))
+        x = np.exp((x - x.max(-1, keepdims=True)) / np.sqrt(D))
+        ref = np.einsum("rhl,lhd->rhd", x / x.sum(-1, keepdims=True), vr.astype(np.float64))
+    for got in (o, whole):
+        got = got.cpu().numpy().astype(np.float32)
+        assert np.isfinite(got).all()
+        assert np.abs(got[rows] - ref).max() <= 2e-3
+    assert (o.float() - whole.float()).abs().max() <= 2e-3
