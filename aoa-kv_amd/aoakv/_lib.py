@@ -63,6 +63,8 @@ SIGNATURES = {
                                      _u32, _u32, _u32, _p, _sz, _p],
     "aoakv_apply_rope_in_place": [_p, _p, _u32, _u32, _u32, _u32, _u32, _f32, _f32, _p],
     "aoakv_rms_norm_forward": [_p, _p, _p, _u32, _u32, _f32, _p],
+    "aoakv_rope_append_kv_cache_prefill": [_p, _p, _p, _u32, _u32, _p, _p, _u32, _u32, _p, _p,
+                                           _p, _p, _u32, _u32, _u32, _u32, _f32, _f32, _p],
     "aoakv_rope_append_kv_cache_decode": [_p, _p, _p, _u32, _u32, _p, _p, _p, _p, _p, _p, _p,
                                           _p, _p, _u32, _u32, _u32, _u32, _f32, _f32, _p],
 }

@@ -152,6 +152,32 @@ def rope_append_kv_cache_decode(q, k, v, kv_data, kv_indptr, kv_indices, kv_last
               layout, float(rope_scale), float(rope_theta), _stream())
 
 
+def rope_append_kv_cache_prefill(q, k, v, kv_data, kv_indices, num_kv_pages: int,
+                                 kv_last_page_len: int, metadata_data, metadata_indices,
+                                 v_log_norm, v_mean, layout: int, rope_scale: float = 1.0,
+                                 rope_theta: float = 1e4):
+    """apply_rope_in_place + append_kv_cache_prefill of a prompt's q [N, Hq, D]
+    and k, v [N, H, D], the sequence's last N tokens (reference calls
+    QuestAttention.py:98-111); one launch at head_dim 128, page_size 16."""
+    for t, n in ((q, "q"), (k, "k"), (v, "v"), (kv_data, "kv_data"),
+                 (metadata_data, "metadata_data"), (v_log_norm, "v_log_norm"), (v_mean, "v_mean")):
+        _need(t, n, torch.float16)
+    _need(kv_indices, "kv_indices", torch.int32)
+    _need(metadata_indices, "metadata_indices", torch.int32)
+    _, S, H, D = cache_dims(kv_data, layout)
+    if k.shape != v.shape or k.dim() != 3 or k.shape[1] != H or k.shape[2] != D:
+        raise ValueError(f"k/v must be [N, {H}, {D}], got {tuple(k.shape)} / {tuple(v.shape)}")
+    if q.dim() != 3 or q.shape[0] != k.shape[0] or q.shape[2] != D:
+        raise ValueError(f"q must be [{k.shape[0]}, Hq, {D}], got {tuple(q.shape)}")
+    if kv_indices.numel() < num_kv_pages:
+        raise ValueError("kv_indices shorter than num_kv_pages")
+    _lib.call("aoakv_rope_append_kv_cache_prefill", q.data_ptr(), k.data_ptr(), v.data_ptr(),
+              k.shape[0], q.shape[1], kv_data.data_ptr(), kv_indices.data_ptr(), num_kv_pages,
+              kv_last_page_len, metadata_data.data_ptr(), metadata_indices.data_ptr(),
+              v_log_norm.data_ptr(), v_mean.data_ptr(), H, D, S, layout, float(rope_scale),
+              float(rope_theta), _stream())
+
+
 def estimate_attn_score(q, scores, metadata_data, metadata_indptr, metadata_indices, kv_indptr,
                         kv_indices, kv_last_page_len, v_log_norm, max_pages: int, layout: int,
                         flags: int = FLAG_VALUE_AWARE):

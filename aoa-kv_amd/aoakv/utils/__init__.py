@@ -66,15 +66,18 @@ def rope_append_kv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                    iController: InferenceController, layer_idx: int,
                    rope_scale: Optional[float] = None, rope_theta: Optional[float] = None):
     """apply_rope_in_place(q, k, seqlen - N) then append_kv(k, v) -- the
-    reference's two calls at QuestAttention.py:98-111 -- with the decode step
-    (N == 1) in one launch.  q and k are left rotated, as the reference leaves
+    reference's two calls at QuestAttention.py:98-111 -- in one launch (a
+    prompt at the shapes ops.rope_append_kv_cache_prefill names).  q and k are left rotated, as the reference leaves
     them.  Call after begin_forward, like append_kv."""
     c = iController
     scale = 1.0 if rope_scale is None else rope_scale
     theta = 1e4 if rope_theta is None else rope_theta
     if k.size(0) > 1:
-        ops.apply_rope_in_place(q, k, c.kv_cache.seqlen - k.size(0), scale, theta)
-        append_kv(k, v, c, layer_idx)
+        ops.rope_append_kv_cache_prefill(
+            q, k, v, c.kv_cache.buf_layer(layer_idx), c.kv_indices_with_last,
+            len(c.kv_cache.indicies), c.kv_cache.last_page_len,
+            c.metadata_cache.buf_layer(layer_idx), c.metadata_indices,
+            c.v_log_norm_layer(layer_idx), c.v_mean_layer(layer_idx), c.layout, scale, theta)
         return
     ops.rope_append_kv_cache_decode(
         q.view(1, -1, c.head_dim), k, v, c.kv_cache.buf_layer(layer_idx),

@@ -24,24 +24,77 @@ constexpr int kHeadsPerWave = 4;
 constexpr int kHeadsPerBlock = 16;
 
 
+// With ROPE the block rows of grid.y past the kv heads' rotate q in place, and
+// k is rotated (in place, and as stored): RoPE and append of a prompt in one
+// pass, where the two launches read k twice.  Bound by HBM: 16000 tokens, 32
+// heads, 944 MB needed: 229 us in two launches (rope_kernel 104, append 118),
+// 187 in one (5.05 TB/s; a 1 GiB copy runs at 5.2).  Small prompts save the
+// launch: 333 tokens 16.7 -> 13.2 us.
+template <bool ROPE>
 __global__ __launch_bounds__(256) void append_prefill_kernel(AppendPrefillArgs a) {
   const uint32_t lane = __lane_id();
   const uint32_t wave = threadIdx.x / kWave;
   const uint32_t row = lane / kLanesPerRow;
   const uint32_t l16 = lane % kLanesPerRow;
-  const uint32_t h = blockIdx.y * kHeadsPerBlock + wave * kHeadsPerWave + row;
+  const uint32_t kv_blocks = (a.H + kHeadsPerBlock - 1) / kHeadsPerBlock;
+  const bool q_block = ROPE && blockIdx.y >= kv_blocks;  // uniform per block
+  const uint32_t h = (q_block ? blockIdx.y - kv_blocks : blockIdx.y) * kHeadsPerBlock +
+                     wave * kHeadsPerWave + row;
   const uint32_t p = a.first_page + blockIdx.x;
-  if (h >= a.H || p >= a.num_pages) return;  // whole rows exit together
 
   const uint32_t S = a.S;
   const uint32_t L = (a.num_pages - 1u) * S + a.last_page_len;
   const uint32_t start = L - a.N;  // first appended position
   const uint32_t e0 = start > p * S ? start - p * S : 0u;
   const uint32_t e1 = (L - p * S) < S ? (L - p * S) : S;
+  const uint32_t n = e1 - e0;
+  const uint32_t d0 = l16 * kVec;
+  const uint32_t tok0 = p * S + e0 - start;  // row of the page's first token in k, v, q
+
+  // cos / sin of the page's tokens for the 64 frequencies, once per block
+  // (the whole 16 heads of each token read them)
+  __shared__ float s_rope[ROPE ? kPageSize : 1][2][kHeadDim / 2];
+  if constexpr (ROPE) {
+    const uint32_t i = threadIdx.x % (kHeadDim / 2);
+    const float f = a.rope_f.f[i];
+    for (uint32_t t = threadIdx.x / (kHeadDim / 2); t < n; t += 256u / (kHeadDim / 2))
+      sincosf((float)(p * S + e0 + t) * f, &s_rope[t][1][i], &s_rope[t][0][i]);
+    __syncthreads();
+  }
+  auto table = [&](uint32_t t) {
+    RopeTable rt;
+    const uint32_t i = d0 % (kHeadDim / 2);
+#pragma unroll
+    for (int j = 0; j < kVec; ++j) {
+      rt.c[j] = s_rope[t][0][i + j];
+      rt.s[j] = s_rope[t][1][i + j];
+    }
+    return rt;
+  };
+  // tokens in flight (with RoPE at 16000 tokens: 2 201 us, 4 194, 8 187, 16
+  // 187; without, 4 and 8 alike)
+  constexpr uint32_t kB = ROPE ? 8 : 4;
+  if constexpr (ROPE) {
+    if (q_block) {
+      if (h >= a.Hq) return;
+      const size_t q_row = (size_t)a.Hq * kHeadDim;
+      f16* q = a.q + tok0 * q_row + (size_t)h * kHeadDim + d0;
+      for (uint32_t i0 = 0; i0 < n; i0 += kB) {
+        H8 x[kB];
+#pragma unroll
+        for (uint32_t u = 0; u < kB; ++u) x[u] = ld16(q + (i0 + u < n ? i0 + u : n - 1u) * q_row);
+#pragma unroll
+        for (uint32_t u = 0; u < kB; ++u)
+          if (i0 + u < n) st16(q + (i0 + u) * q_row, rope_row(x[u], table(i0 + u), l16));
+      }
+      return;
+    }
+  }
+  if (h >= a.H) return;  // whole rows exit together
+
   const uint32_t phys = (uint32_t)a.kv_indices[p];
   const uint32_t mpage = (uint32_t)a.meta_indices[p / S];
   const uint32_t ment = p % S;
-  const uint32_t d0 = l16 * kVec;
 
   f16* kmax_p = a.meta + elem_off(a.g, mpage, 0, h, ment) + d0;
   f16* kmin_p = a.meta + elem_off(a.g, mpage, 1, h, ment) + d0;
@@ -64,43 +117,51 @@ __global__ __launch_bounds__(256) void append_prefill_kernel(AppendPrefillArgs a
   }
 
   const size_t in_row = (size_t)a.H * kHeadDim;
-  const f16* kin = a.k + (size_t)(p * S + e0 - start) * in_row + (size_t)h * kHeadDim + d0;
-  const f16* vin = a.v + (size_t)(p * S + e0 - start) * in_row + (size_t)h * kHeadDim + d0;
+  f16* kin = a.k + tok0 * in_row + (size_t)h * kHeadDim + d0;
+  const f16* vin = a.v + tok0 * in_row + (size_t)h * kHeadDim + d0;
   f16* kout = a.kv + elem_off(a.g, phys, 0, h, e0) + d0;
   f16* vout = a.kv + elem_off(a.g, phys, 1, h, e0) + d0;
 
-  const uint32_t n = e1 - e0;
-  if (e0 == 0u) {
-    // page filled from empty: V̄ = mean over its tokens (compute_page_v_mean)
-#pragma unroll 4
-    for (uint32_t i = 0; i < n; ++i) {
-      H8 kk = ld16(kin + i * in_row);
-      H8 vv = ld16(vin + i * in_row);
+  // kB tokens' loads go out together (the in-place stores of k would
+  // otherwise hold back the next token's loads)
+  for (uint32_t i0 = 0; i0 < n; i0 += kB) {
+    H8 kk[kB], vv[kB];
+#pragma unroll
+    for (uint32_t u = 0; u < kB; ++u) {
+      const uint32_t i = i0 + u < n ? i0 + u : n - 1u;
+      kk[u] = ld16(kin + i * in_row);
+      vv[u] = ld16(vin + i * in_row);
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kB; ++u) {
+      const uint32_t i = i0 + u;
+      if (i >= n) break;
+      if constexpr (ROPE) {
+        kk[u] = rope_row(kk[u], table(i), l16);
+        st16(kin + i * in_row, kk[u]);
+      }
 #pragma unroll
       for (int j = 0; j < kVec; ++j) {
-        kmax.v[j] = kk.v[j] > kmax.v[j] ? kk.v[j] : kmax.v[j];
-        kmin.v[j] = kk.v[j] < kmin.v[j] ? kk.v[j] : kmin.v[j];
-        vsum[j] = vsum[j] + (float)vv.v[j];
+        kmax.v[j] = kk[u].v[j] > kmax.v[j] ? kk[u].v[j] : kmax.v[j];
+        kmin.v[j] = kk[u].v[j] < kmin.v[j] ? kk[u].v[j] : kmin.v[j];
       }
-      st16(kout + (size_t)i * a.g.tok, kk);
-      st16(vout + (size_t)i * a.g.tok, vv);
+      if (e0 == 0u) {
+        // page filled from empty: V̄ = mean over its tokens (compute_page_v_mean)
+#pragma unroll
+        for (int j = 0; j < kVec; ++j) vsum[j] = vsum[j] + (float)vv[u].v[j];
+      } else {
+        // tokens added to a page that already holds e0 tokens: running mean
+#pragma unroll
+        for (int j = 0; j < kVec; ++j)
+          vbar.v[j] = running_mean(vbar.v[j], vv[u].v[j], e0 + i);
+      }
+      st16(kout + (size_t)i * a.g.tok, kk[u]);
+      st16(vout + (size_t)i * a.g.tok, vv[u]);
     }
+  }
+  if (e0 == 0u) {
 #pragma unroll
     for (int j = 0; j < kVec; ++j) vbar.v[j] = r16(vsum[j] / (float)n);
-  } else {
-    // tokens added to a page that already holds e0 tokens: running mean
-    for (uint32_t i = 0; i < n; ++i) {
-      H8 kk = ld16(kin + i * in_row);
-      H8 vv = ld16(vin + i * in_row);
-#pragma unroll
-      for (int j = 0; j < kVec; ++j) {
-        kmax.v[j] = kk.v[j] > kmax.v[j] ? kk.v[j] : kmax.v[j];
-        kmin.v[j] = kk.v[j] < kmin.v[j] ? kk.v[j] : kmin.v[j];
-        vbar.v[j] = running_mean(vbar.v[j], vv.v[j], e0 + i);
-      }
-      st16(kout + (size_t)i * a.g.tok, kk);
-      st16(vout + (size_t)i * a.g.tok, vv);
-    }
   }
   st16(kmax_p, kmax);
   st16(kmin_p, kmin);
@@ -191,8 +252,14 @@ hipError_t launch_append_prefill(const AppendPrefillArgs& a, hipStream_t s) {
   const uint32_t first_page = (L - a.N) / a.S;
   AppendPrefillArgs b = a;
   b.first_page = first_page;
-  dim3 grid(a.num_pages - first_page, (a.H + kHeadsPerBlock - 1) / kHeadsPerBlock);
-  hipLaunchKernelGGL(append_prefill_kernel, grid, dim3(256), 0, s, b);
+  const uint32_t kv_blocks = (a.H + kHeadsPerBlock - 1) / kHeadsPerBlock;
+  dim3 grid(a.num_pages - first_page, kv_blocks);
+  if (a.q != nullptr) {
+    grid.y += (a.Hq + kHeadsPerBlock - 1) / kHeadsPerBlock;
+    hipLaunchKernelGGL(append_prefill_kernel<true>, grid, dim3(256), 0, s, b);
+  } else {
+    hipLaunchKernelGGL(append_prefill_kernel<false>, grid, dim3(256), 0, s, b);
+  }
   return hipGetLastError();
 }
 

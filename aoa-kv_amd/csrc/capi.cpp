@@ -266,27 +266,25 @@ const char* aoakv_last_error(void) { return g_err.c_str(); }
 
 const char* aoakv_version(void) { return "aoakv-mi355x 0.1 (gfx950)"; }
 
-int aoakv_append_kv_cache_prefill(const void* k, const void* v, uint32_t num_new_tokens,
-                                  void* kv_data, const int32_t* kv_indices,
-                                  uint32_t num_kv_pages, uint32_t kv_last_page_len,
-                                  void* metadata_data, const int32_t* metadata_indices,
-                                  void* v_log_norm, void* v_mean, uint32_t num_heads,
-                                  uint32_t head_dim, uint32_t page_size, uint32_t layout,
-                                  void* stream) {
+static int fill_append_prefill(aoakv::AppendPrefillArgs& a, void* k, const void* v,
+                               uint32_t num_new_tokens, void* kv_data, const int32_t* kv_indices,
+                               uint32_t num_kv_pages, uint32_t kv_last_page_len,
+                               void* metadata_data, const int32_t* metadata_indices,
+                               void* v_log_norm, void* v_mean, uint32_t num_heads,
+                               uint32_t head_dim, uint32_t page_size, uint32_t layout,
+                               const char* fn) {
   if (int e = check_shape(head_dim, page_size, layout, num_heads)) return e;
   REQUIRE(k && v && kv_data && kv_indices && metadata_data && metadata_indices && v_log_norm &&
               v_mean,
-          "append_kv_cache_prefill: null pointer argument");
-  REQUIRE(num_kv_pages >= 1u, "append_kv_cache_prefill: num_kv_pages must be >= 1");
+          "%s: null pointer argument", fn);
+  REQUIRE(num_kv_pages >= 1u, "%s: num_kv_pages must be >= 1", fn);
   REQUIRE(kv_last_page_len >= 1u && kv_last_page_len <= page_size,
-          "append_kv_cache_prefill: kv_last_page_len %u not in [1, %u]", kv_last_page_len,
-          page_size);
+          "%s: kv_last_page_len %u not in [1, %u]", fn, kv_last_page_len, page_size);
   const uint64_t L = (uint64_t)(num_kv_pages - 1u) * page_size + kv_last_page_len;
   REQUIRE(num_new_tokens >= 1u && num_new_tokens <= L,
-          "append_kv_cache_prefill: %u new tokens but the cache holds %llu", num_new_tokens,
+          "%s: %u new tokens but the cache holds %llu", fn, num_new_tokens,
           (unsigned long long)L);
-  aoakv::AppendPrefillArgs a{};
-  a.k = static_cast<const aoakv::f16*>(k);
+  a.k = static_cast<aoakv::f16*>(k);
   a.v = static_cast<const aoakv::f16*>(v);
   a.kv = static_cast<aoakv::f16*>(kv_data);
   a.kv_indices = kv_indices;
@@ -300,11 +298,33 @@ int aoakv_append_kv_cache_prefill(const void* k, const void* v, uint32_t num_new
   a.num_pages = num_kv_pages;
   a.last_page_len = kv_last_page_len;
   a.g = aoakv::make_geom(layout, num_heads, page_size, head_dim);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  return hip_status(aoakv::tuned_shape(head_dim, page_size)
+  return AOAKV_OK;
+}
+
+static int launch_append_prefill(const aoakv::AppendPrefillArgs& a, uint32_t head_dim,
+                                 hipStream_t s, const char* fn) {
+  return hip_status(aoakv::tuned_shape(head_dim, a.S)
                         ? aoakv::launch_append_prefill(a, s)
                         : aoakv::launch_gen_append_prefill(a, head_dim, s),
-                    "append_kv_cache_prefill");
+                    fn);
+}
+
+int aoakv_append_kv_cache_prefill(const void* k, const void* v, uint32_t num_new_tokens,
+                                  void* kv_data, const int32_t* kv_indices,
+                                  uint32_t num_kv_pages, uint32_t kv_last_page_len,
+                                  void* metadata_data, const int32_t* metadata_indices,
+                                  void* v_log_norm, void* v_mean, uint32_t num_heads,
+                                  uint32_t head_dim, uint32_t page_size, uint32_t layout,
+                                  void* stream) {
+  aoakv::AppendPrefillArgs a{};
+  // k is only read without RoPE
+  if (int e = fill_append_prefill(a, const_cast<void*>(k), v, num_new_tokens, kv_data, kv_indices,
+                                  num_kv_pages, kv_last_page_len, metadata_data, metadata_indices,
+                                  v_log_norm, v_mean, num_heads, head_dim, page_size, layout,
+                                  "append_kv_cache_prefill"))
+    return e;
+  return launch_append_prefill(a, head_dim, static_cast<hipStream_t>(stream),
+                               "append_kv_cache_prefill");
 }
 
 int aoakv_append_kv_cache_decode(const void* k, const void* v, uint32_t batch_size,
@@ -438,6 +458,49 @@ int aoakv_rope_append_kv_cache_decode(void* q, void* k, const void* v, uint32_t 
                         ? aoakv::launch_append_decode(a, batch_size, s)
                         : aoakv::launch_gen_append_decode(a, batch_size, head_dim, s),
                     "rope_append_kv_cache_decode");
+}
+
+int aoakv_rope_append_kv_cache_prefill(void* q, void* k, const void* v, uint32_t num_new_tokens,
+                                       uint32_t num_qo_heads, void* kv_data,
+                                       const int32_t* kv_indices, uint32_t num_kv_pages,
+                                       uint32_t kv_last_page_len, void* metadata_data,
+                                       const int32_t* metadata_indices, void* v_log_norm,
+                                       void* v_mean, uint32_t num_heads, uint32_t head_dim,
+                                       uint32_t page_size, uint32_t layout, float rope_scale,
+                                       float rope_theta, void* stream) {
+  const char* fn = "rope_append_kv_cache_prefill";
+  aoakv::AppendPrefillArgs a{};
+  if (int e = fill_append_prefill(a, k, v, num_new_tokens, kv_data, kv_indices, num_kv_pages,
+                                  kv_last_page_len, metadata_data, metadata_indices, v_log_norm,
+                                  v_mean, num_heads, head_dim, page_size, layout, fn))
+    return e;
+  REQUIRE(q, "%s: null pointer argument", fn);
+  REQUIRE(num_qo_heads >= 1u && num_qo_heads <= 256u, "%s: num_qo_heads %u out of range [1, 256]",
+          fn, num_qo_heads);
+  const uint64_t L = (uint64_t)(num_kv_pages - 1u) * page_size + kv_last_page_len;
+  REQUIRE(L <= (1ull << 24), "%s: positions up to %llu exceed 2^24 (fp32 positions)", fn,
+          (unsigned long long)L);
+  if (int e = check_rope(rope_scale, rope_theta, fn)) return e;
+  // one pass for the tuned shape; k and v (or q) sharing memory keep the
+  // order of the two calls, whose second reads what the first rotated
+  const size_t row = (size_t)num_new_tokens * head_dim * sizeof(aoakv::f16);
+  auto apart = [](const void* x, size_t nx, const void* y, size_t ny) {
+    const uintptr_t a0 = (uintptr_t)x, b0 = (uintptr_t)y;
+    return a0 + nx <= b0 || b0 + ny <= a0;
+  };
+  if (aoakv::tuned_shape(head_dim, page_size) && apart(k, row * num_heads, v, row * num_heads) &&
+      apart(q, row * num_qo_heads, k, row * num_heads) &&
+      apart(q, row * num_qo_heads, v, row * num_heads)) {
+    a.q = static_cast<aoakv::f16*>(q);
+    a.Hq = num_qo_heads;
+    a.rope_f = aoakv::rope_freqs(rope_scale, rope_theta, head_dim);
+  } else if (int e = aoakv_apply_rope_in_place(q, k, num_new_tokens,
+                                               (uint32_t)L - num_new_tokens, num_qo_heads,
+                                               num_heads, head_dim, rope_scale, rope_theta,
+                                               stream)) {
+    return e;
+  }
+  return launch_append_prefill(a, head_dim, static_cast<hipStream_t>(stream), fn);
 }
 
 static int fill_estimate(aoakv::EstimateArgs& a, const void* q, float* scores,

@@ -56,7 +56,7 @@ struct RopeFreqs {
 RopeFreqs rope_freqs(float rope_scale, float rope_theta, uint32_t head_dim = kHeadDim);
 
 struct AppendPrefillArgs {
-  const f16* k;            // [N, H, D]
+  f16* k;                  // [N, H, D] (rotated in place with q)
   const f16* v;            // [N, H, D]
   f16* kv;                 // paged cache of the layer
   const int32_t* kv_indices;
@@ -66,6 +66,11 @@ struct AppendPrefillArgs {
   f16* v_mean;             // [max_pages, H, D]
   uint32_t N, H, S, num_pages, last_page_len, first_page;
   PageGeom g;
+  // fused RoPE (q != nullptr): q [N, Hq, D] and k rotated in place, k stored
+  // rotated
+  f16* q;
+  uint32_t Hq;
+  RopeFreqs rope_f;
 };
 
 struct AppendDecodeArgs {

@@ -220,6 +220,22 @@ int aoakv_rope_append_kv_cache_decode(void* q, void* k, const void* v, uint32_t 
                                       float rope_theta, void* stream);
 
 /*
+ * A prompt's RoPE and bulk append: aoakv_apply_rope_in_place on q
+ * [N, num_qo_heads, D] and k [N, num_heads, D] at the sequence's last N
+ * positions, then aoakv_append_kv_cache_prefill of the rotated k and v.  Same
+ * results, bit for bit, as the two calls; one launch with head_dim 128 and
+ * page_size 16 when q, k and v do not overlap.
+ */
+int aoakv_rope_append_kv_cache_prefill(void* q, void* k, const void* v, uint32_t num_new_tokens,
+                                       uint32_t num_qo_heads, void* kv_data,
+                                       const int32_t* kv_indices, uint32_t num_kv_pages,
+                                       uint32_t kv_last_page_len, void* metadata_data,
+                                       const int32_t* metadata_indices, void* v_log_norm,
+                                       void* v_mean, uint32_t num_heads, uint32_t head_dim,
+                                       uint32_t page_size, uint32_t layout, float rope_scale,
+                                       float rope_theta, void* stream);
+
+/*
  * Page scores of every page of every sequence.  Replaces estimate_attn_score
  * (reference bsk_ops.h:41-51, estimate.cu:6-90, decode_attn.cuh:145-199,
  * 276-443); follows filter_util.py:269-380,968-1018:

@@ -169,3 +169,56 @@ def test_fused_rope_append_equals_rope_then_append(layout, L0):
     assert np.array_equal(bits(pf), bits(st.page_filters))
     assert np.array_equal(bits(vm), bits(st.v_mean))
     assert np.array_equal(bits(lvn.T[None]), bits(sim.log_v_norm(st.v_mean)))
+
+
+@pytest.mark.parametrize("L0,N,Hq,H,d,page,layout", [
+    (0, 17, 20, 20, 128, 16, HND),     # heads past a block of 16, a one-token last page
+    (0, 2, 4, 4, 128, 16, NHD),        # fewer tokens than are loaded together
+    (7, 64, 32, 8, 128, 16, NHD),      # the first page holds tokens already, GQA
+    (48, 25, 8, 8, 128, 16, HND),      # starts a page; 9 tokens in the last
+    (15, 1009, 16, 2, 128, 16, HND),   # one token in the first page
+    (5, 40, 8, 4, 64, 8, NHD),         # two launches: another shape
+])
+def test_fused_rope_append_of_a_prompt_equals_rope_then_append(L0, N, Hq, H, d, page, layout):
+    """aoakv_rope_append_kv_cache_prefill vs aoakv_apply_rope_in_place +
+    aoakv_append_kv_cache_prefill on a twin cache: the same bits everywhere."""
+    from aoakv.utils import InferenceController, append_kv, apply_rope_in_place, rope_append_kv
+    _say(f"[rope-append prompt] {L0}+{N} heads {Hq}/{H} x {d} page {page} layout {layout}")
+    got = []
+    for fused in (True, False):
+        c = InferenceController(1, Hq, d, page, 8, L0 + N + page, torch.float16, DEV,
+                                layout=layout, num_kv_heads=H, shuffle_seed=9)
+        for t in (c.kv_cache.pool.buf, c.metadata_cache.pool.buf):
+            t.zero_()
+        if L0:
+            c.prepare_metadata(L0)
+            c.begin_forward(L0)
+            k0, v0 = (torch.from_numpy(randn16(s, (L0, H, d))).to(DEV) for s in (1, 2))
+            append_kv(k0, v0, c, 0)
+        c.prepare_metadata(N)
+        c.begin_forward(N)
+        q, k, v = (torch.from_numpy(randn16(s, (N, h, d))).to(DEV)
+                   for s, h in ((3, Hq), (4, H), (5, H)))
+        if fused:
+            rope_append_kv(q, k, v, c, 0, rope_scale=2.0, rope_theta=5e5)
+        else:
+            apply_rope_in_place(q, k, L0, 2.0, 5e5)
+            append_kv(k, v, c, 0)
+        got.append([t.cpu() for t in (q, k, v, c.kv_cache.buf_layer(0),
+                                      c.metadata_cache.buf_layer(0), c.v_mean_layer(0),
+                                      c.v_log_norm_layer(0))])
+    for name, x, y in zip(("q", "k", "v", "cache", "Kmax/Kmin", "V mean", "log-norm"), *got):
+        assert np.array_equal(bits(x.numpy()), bits(y.numpy())), name
+
+
+def test_fused_rope_append_of_a_prompt_with_shared_k_and_v():
+    """v is k's own tensor: the append reads it rotated, as the two calls do."""
+    from aoakv.utils import InferenceController, rope_append_kv
+    c = InferenceController(1, 4, D, S, 8, 64, torch.float16, DEV)
+    c.prepare_metadata(33)
+    c.begin_forward(33)
+    q, k = (torch.from_numpy(randn16(s, (33, 4, D))).to(DEV) for s in (1, 2))
+    rope_append_kv(q, k, k, c, 0)
+    K, V = read_kv(c.kv_cache.buf_layer(0), HND, c.kv_cache.indicies, 33)
+    assert np.array_equal(bits(K), bits(V))
+    assert np.array_equal(bits(K[0].transpose(1, 0, 2)), bits(k.cpu().numpy()))
