@@ -24,6 +24,9 @@ SRC_DIR = os.path.join(os.path.dirname(PKG_DIR), "csrc")
 OBJ_DIR = os.path.join(os.path.dirname(PKG_DIR), "_build")
 LIB = os.path.join(PKG_DIR, "libaoakv.so")
 TIMELINE_LIB = os.path.join(PKG_DIR, "libaoakv_timeline.so")
+# the torch-tensor wrappers in C++ (csrc/host.cpp), a Python extension module
+HOST_LIB = os.path.join(PKG_DIR, "_host.so")
+HOST_SOURCE = "host.cpp"
 # build record beside the library (travels with it; the GPU box has no .git)
 BUILDINFO = os.path.join(PKG_DIR, "libaoakv.buildinfo.json")
 SOURCES = ["append.hip", "decode.hip", "prefill.hip", "generic.hip", "norm.hip", "capi.cpp"]
@@ -116,10 +119,36 @@ def _link(lib: str, obj_dir: str, defines=()) -> str:
     return lib
 
 
+def build_host() -> str:
+    """Compile aoakv._host (host code only: torch's headers, no kernels)."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    tmp = HOST_LIB + ".tmp"
+    lib_dirs = [os.path.join(os.path.dirname(torch.__file__), "lib")]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
+           "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[f"-isystem{d}" for d in (sysconfig.get_paths()["include"],
+                                      *cpp_extension.include_paths(),
+                                      os.path.join(os.path.dirname(os.path.dirname(HIPCC)),
+                                                   "include"))],
+           os.path.join(SRC_DIR, HOST_SOURCE), "-o", tmp, *[f"-L{d}" for d in lib_dirs],
+           "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{HOST_SOURCE} failed:\n{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, HOST_LIB)
+    return HOST_LIB
+
+
 def build(verbose: bool = True, timeline: bool = False) -> str:
-    """Compile every source for gfx950 and link libaoakv.so.  Always rebuilds.
-    With timeline, also the profiling build libaoakv_timeline.so."""
+    """Compile every source for gfx950 and link libaoakv.so, then the Python
+    extension module.  Always rebuilds.  With timeline, also the profiling
+    build libaoakv_timeline.so."""
     _link(LIB, OBJ_DIR)
+    build_host()
     write_buildinfo()
     if verbose:
         print(f"built {LIB} ({os.path.getsize(LIB)} bytes)")

@@ -3,6 +3,8 @@
 Each function checks dtypes, devices and shapes, then calls the C ABI with
 raw device pointers on torch's current HIP stream.  Tensors are never
 copied or converted here: a wrong dtype / layout is an error, not a cast.
+The calls of the append, decode and prefill paths do this in C++ (aoakv._host,
+csrc/host.cpp), where a call's checks cost more than a short kernel.
 """
 from __future__ import annotations
 
@@ -11,9 +13,11 @@ from typing import Optional
 
 import torch
 
-from . import _lib
+from . import _host, _lib
 from ._lib import (FLAG_FIXED, FLAG_GROUPED_DECODE, FLAG_QUEST_KERNEL,  # noqa: F401
                    FLAG_SINGLE_LAUNCH, FLAG_VALUE_AWARE)  # (re-exported)
+
+_host.bind(_lib.loaded_path(), _lib.AoakvError, ctypes.ArgumentError)
 
 NHD = 0
 HND = 1
@@ -55,20 +59,8 @@ def cache_dims(kv_data: torch.Tensor, layout: int):
 def append_kv_cache_prefill(k, v, kv_data, kv_indices, num_kv_pages: int, kv_last_page_len: int,
                             metadata_data, metadata_indices, v_log_norm, v_mean, layout: int):
     """Reference: quest/ops/csrc/page.cu:107-222 (append_kv_cache_prefill)."""
-    for t, n in ((k, "k"), (v, "v"), (kv_data, "kv_data"), (metadata_data, "metadata_data"),
-                 (v_log_norm, "v_log_norm"), (v_mean, "v_mean")):
-        _need(t, n, torch.float16)
-    _need(kv_indices, "kv_indices", torch.int32)
-    _need(metadata_indices, "metadata_indices", torch.int32)
-    _, S, H, D = cache_dims(kv_data, layout)
-    if k.shape != v.shape or k.dim() != 3 or k.shape[1] != H or k.shape[2] != D:
-        raise ValueError(f"k/v must be [N, {H}, {D}], got {tuple(k.shape)} / {tuple(v.shape)}")
-    if kv_indices.numel() < num_kv_pages:
-        raise ValueError("kv_indices shorter than num_kv_pages")
-    _lib.call("aoakv_append_kv_cache_prefill", k.data_ptr(), v.data_ptr(), k.shape[0],
-              kv_data.data_ptr(), kv_indices.data_ptr(), num_kv_pages, kv_last_page_len,
-              metadata_data.data_ptr(), metadata_indices.data_ptr(), v_log_norm.data_ptr(),
-              v_mean.data_ptr(), H, D, S, layout, _stream())
+    _host.append_kv_cache_prefill(k, v, kv_data, kv_indices, num_kv_pages, kv_last_page_len,
+                                  metadata_data, metadata_indices, v_log_norm, v_mean, layout)
 
 
 def append_kv_cache_decode(k, v, kv_data, kv_indptr, kv_indices, kv_last_page_len,
@@ -76,23 +68,9 @@ def append_kv_cache_decode(k, v, kv_data, kv_indptr, kv_indices, kv_last_page_le
                            layout: int):
     """Reference: quest/ops/csrc/page.cu:6-105 (append_kv_cache_decode); k, v
     are [B, H, D], one new token per sequence."""
-    for t, n in ((k, "k"), (v, "v"), (kv_data, "kv_data"), (metadata_data, "metadata_data"),
-                 (v_log_norm, "v_log_norm"), (v_mean, "v_mean")):
-        _need(t, n, torch.float16)
-    for t, n in ((kv_indptr, "kv_indptr"), (kv_indices, "kv_indices"),
-                 (kv_last_page_len, "kv_last_page_len"), (metadata_indptr, "metadata_indptr"),
-                 (metadata_indices, "metadata_indices")):
-        _need(t, n, torch.int32)
-    _, S, H, D = cache_dims(kv_data, layout)
-    B = k.shape[0]
-    if k.shape != (B, H, D) or v.shape != (B, H, D):
-        raise ValueError(f"k/v must be [B, {H}, {D}]")
-    if kv_indptr.numel() != B + 1 or kv_last_page_len.numel() != B or metadata_indptr.numel() != B + 1:
-        raise ValueError("indptr / last_page_len sizes do not match the batch")
-    _lib.call("aoakv_append_kv_cache_decode", k.data_ptr(), v.data_ptr(), B, kv_data.data_ptr(),
-              kv_indptr.data_ptr(), kv_indices.data_ptr(), kv_last_page_len.data_ptr(),
-              metadata_data.data_ptr(), metadata_indptr.data_ptr(), metadata_indices.data_ptr(),
-              v_log_norm.data_ptr(), v_mean.data_ptr(), H, D, S, layout, _stream())
+    _host.append_kv_cache_decode(k, v, kv_data, kv_indptr, kv_indices, kv_last_page_len,
+                                 metadata_data, metadata_indptr, metadata_indices, v_log_norm,
+                                 v_mean, layout)
 
 
 def apply_rope_in_place(q, k, past_kv_len: int, rope_scale: float = 1.0,
@@ -113,15 +91,7 @@ def rms_norm_forward(input, weight, output, epsilon: float):
     """Reference: quest/ops/csrc/rms_norm.cu:185-213 (bsk_ops.h:29): RMSNorm of
     input [..., n] fp16 (rows over the leading dims) with weight [n] into
     output (input's shape; may be input itself)."""
-    _need(input, "input", torch.float16)
-    _need(weight, "weight", torch.float16)
-    _need(output, "output", torch.float16)
-    n = input.shape[-1]
-    if weight.shape != (n,) or output.shape != input.shape:
-        raise ValueError(f"weight must be [{n}] and output {tuple(input.shape)}, got "
-                         f"{tuple(weight.shape)} / {tuple(output.shape)}")
-    _lib.call("aoakv_rms_norm_forward", input.data_ptr(), weight.data_ptr(), output.data_ptr(),
-              input.numel() // n, n, float(epsilon), _stream())
+    _host.rms_norm_forward(input, weight, output, float(epsilon))
 
 
 def rope_append_kv_cache_decode(q, k, v, kv_data, kv_indptr, kv_indices, kv_last_page_len,
@@ -131,25 +101,10 @@ def rope_append_kv_cache_decode(q, k, v, kv_data, kv_indptr, kv_indices, kv_last
     """apply_rope_in_place + append_kv_cache_decode in one launch: q [B, Hq, D]
     and k [B, H, D] rotated in place at each sequence's new position, then k, v
     appended with metadata (reference calls QuestAttention.py:98-111)."""
-    for t, n in ((q, "q"), (k, "k"), (v, "v"), (kv_data, "kv_data"),
-                 (metadata_data, "metadata_data"), (v_log_norm, "v_log_norm"), (v_mean, "v_mean")):
-        _need(t, n, torch.float16)
-    for t, n in ((kv_indptr, "kv_indptr"), (kv_indices, "kv_indices"),
-                 (kv_last_page_len, "kv_last_page_len"), (metadata_indptr, "metadata_indptr"),
-                 (metadata_indices, "metadata_indices")):
-        _need(t, n, torch.int32)
-    _, S, H, D = cache_dims(kv_data, layout)
-    B = k.shape[0]
-    if k.shape != (B, H, D) or v.shape != (B, H, D) or q.dim() != 3 or q.shape[0] != B \
-            or q.shape[2] != D:
-        raise ValueError(f"q must be [B, Hq, {D}], k/v [B, {H}, {D}]")
-    if kv_indptr.numel() != B + 1 or kv_last_page_len.numel() != B or metadata_indptr.numel() != B + 1:
-        raise ValueError("indptr / last_page_len sizes do not match the batch")
-    _lib.call("aoakv_rope_append_kv_cache_decode", q.data_ptr(), k.data_ptr(), v.data_ptr(), B,
-              q.shape[1], kv_data.data_ptr(), kv_indptr.data_ptr(), kv_indices.data_ptr(),
-              kv_last_page_len.data_ptr(), metadata_data.data_ptr(), metadata_indptr.data_ptr(),
-              metadata_indices.data_ptr(), v_log_norm.data_ptr(), v_mean.data_ptr(), H, D, S,
-              layout, float(rope_scale), float(rope_theta), _stream())
+    _host.rope_append_kv_cache_decode(q, k, v, kv_data, kv_indptr, kv_indices, kv_last_page_len,
+                                      metadata_data, metadata_indptr, metadata_indices,
+                                      v_log_norm, v_mean, layout, float(rope_scale),
+                                      float(rope_theta))
 
 
 def rope_append_kv_cache_prefill(q, k, v, kv_data, kv_indices, num_kv_pages: int,
@@ -159,23 +114,10 @@ def rope_append_kv_cache_prefill(q, k, v, kv_data, kv_indices, num_kv_pages: int
     """apply_rope_in_place + append_kv_cache_prefill of a prompt's q [N, Hq, D]
     and k, v [N, H, D], the sequence's last N tokens (reference calls
     QuestAttention.py:98-111); one launch at head_dim 128, page_size 16."""
-    for t, n in ((q, "q"), (k, "k"), (v, "v"), (kv_data, "kv_data"),
-                 (metadata_data, "metadata_data"), (v_log_norm, "v_log_norm"), (v_mean, "v_mean")):
-        _need(t, n, torch.float16)
-    _need(kv_indices, "kv_indices", torch.int32)
-    _need(metadata_indices, "metadata_indices", torch.int32)
-    _, S, H, D = cache_dims(kv_data, layout)
-    if k.shape != v.shape or k.dim() != 3 or k.shape[1] != H or k.shape[2] != D:
-        raise ValueError(f"k/v must be [N, {H}, {D}], got {tuple(k.shape)} / {tuple(v.shape)}")
-    if q.dim() != 3 or q.shape[0] != k.shape[0] or q.shape[2] != D:
-        raise ValueError(f"q must be [{k.shape[0]}, Hq, {D}], got {tuple(q.shape)}")
-    if kv_indices.numel() < num_kv_pages:
-        raise ValueError("kv_indices shorter than num_kv_pages")
-    _lib.call("aoakv_rope_append_kv_cache_prefill", q.data_ptr(), k.data_ptr(), v.data_ptr(),
-              k.shape[0], q.shape[1], kv_data.data_ptr(), kv_indices.data_ptr(), num_kv_pages,
-              kv_last_page_len, metadata_data.data_ptr(), metadata_indices.data_ptr(),
-              v_log_norm.data_ptr(), v_mean.data_ptr(), H, D, S, layout, float(rope_scale),
-              float(rope_theta), _stream())
+    _host.rope_append_kv_cache_prefill(q, k, v, kv_data, kv_indices, num_kv_pages,
+                                       kv_last_page_len, metadata_data, metadata_indices,
+                                       v_log_norm, v_mean, layout, float(rope_scale),
+                                       float(rope_theta))
 
 
 def estimate_attn_score(q, scores, metadata_data, metadata_indptr, metadata_indices, kv_indptr,
@@ -183,23 +125,9 @@ def estimate_attn_score(q, scores, metadata_data, metadata_indptr, metadata_indi
                         flags: int = FLAG_VALUE_AWARE):
     """Reference: quest/ops/csrc/estimate.cu:6-90.  q [B, Hq, D] fp16 ->
     scores [B, Hkv, stride] fp32 (stride = scores.shape[-1])."""
-    _need(q, "q", torch.float16)
-    _need(scores, "scores", torch.float32)
-    _need(metadata_data, "metadata_data", torch.float16)
-    for t, n in ((metadata_indptr, "metadata_indptr"), (metadata_indices, "metadata_indices"),
-                 (kv_indptr, "kv_indptr"), (kv_indices, "kv_indices"),
-                 (kv_last_page_len, "kv_last_page_len")):
-        _need(t, n, torch.int32)
-    if flags & FLAG_VALUE_AWARE:
-        _need(v_log_norm, "v_log_norm", torch.float16)
-    _, S, Hkv, D = cache_dims(metadata_data, layout)
-    B, Hq, Dq = q.shape
-    if Dq != D or scores.dim() != 3 or scores.shape[0] != B or scores.shape[1] != Hkv:
-        raise ValueError(f"scores must be [B, {Hkv}, >= max_pages]")
-    _lib.call("aoakv_estimate_attn_score", q.data_ptr(), scores.data_ptr(), scores.shape[2],
-              metadata_data.data_ptr(), metadata_indptr.data_ptr(), metadata_indices.data_ptr(),
-              kv_indptr.data_ptr(), kv_indices.data_ptr(), kv_last_page_len.data_ptr(),
-              _ptr(v_log_norm), B, max_pages, Hq, Hkv, D, S, layout, flags, _stream())
+    _host.estimate_attn_score(q, scores, metadata_data, metadata_indptr, metadata_indices,
+                              kv_indptr, kv_indices, kv_last_page_len, v_log_norm, max_pages,
+                              layout, flags)
 
 
 def topk_filtering(scores, kv_indptr, kv_indices, kv_last_page_len, token_budget: int, sel_pages,
@@ -209,26 +137,8 @@ def topk_filtering(scores, kv_indptr, kv_indices, kv_last_page_len, token_budget
     (physical page ids, ascending logical order).  ``workspace``: a decode
     workspace whose error word receives WS_ERR_TRUNCATED when a page table
     holds more pages than a score row (None: not reported)."""
-    _need(scores, "scores", torch.float32)
-    _need(sel_pages, "sel_pages", torch.int32)
-    for t, n in ((kv_indptr, "kv_indptr"), (kv_indices, "kv_indices"),
-                 (kv_last_page_len, "kv_last_page_len")):
-        _need(t, n, torch.int32)
-    if token_budgets is not None:
-        _need(token_budgets, "token_budgets", torch.int32)
-    B, Hkv, stride = scores.shape
-    if sel_pages.dim() != 3 or sel_pages.shape[:2] != (B, Hkv):
-        raise ValueError("sel_pages must be [B, Hkv, k_max]")
-    err = None
-    if workspace is not None:
-        _need(workspace, "workspace", torch.uint8)
-        if workspace.numel() < 12:
-            raise ValueError("workspace too small to hold the error word")
-        err = workspace.data_ptr() + 4 * WS_ERR_WORD
-    _lib.call("aoakv_topk_filtering", scores.data_ptr(), stride, kv_indptr.data_ptr(),
-              kv_indices.data_ptr(), kv_last_page_len.data_ptr(), token_budget,
-              _ptr(token_budgets), sel_pages.data_ptr(), sel_pages.shape[2], B, Hkv, page_size,
-              flags, err, _stream())
+    _host.topk_filtering(scores, kv_indptr, kv_indices, kv_last_page_len, token_budget, sel_pages,
+                         page_size, flags, token_budgets, workspace)
 
 
 def decode_workspace(batch: int, num_qo_heads: int, num_kv_heads: int, max_sel_pages: int,
@@ -287,28 +197,9 @@ def decode_sparse_attn(q, o, kv_data, kv_indptr, kv_indices, kv_last_page_len, s
     """Reference: quest/ops/csrc/approx_attn.cu:68-151.  sel_pages None = dense.
     ``flags`` = FLAG_QUEST_KERNEL: sel_pages rows hold the pages chosen
     besides the last page, which is attended as well."""
-    _need(q, "q", torch.float16)
-    _need(o, "o", torch.float16)
-    _need(kv_data, "kv_data", torch.float16)
-    _need(workspace, "workspace", torch.uint8)
-    for t, n in ((kv_indptr, "kv_indptr"), (kv_indices, "kv_indices"),
-                 (kv_last_page_len, "kv_last_page_len")):
-        _need(t, n, torch.int32)
-    if sel_pages is not None:
-        _need(sel_pages, "sel_pages", torch.int32)
-    if token_budgets is not None:
-        _need(token_budgets, "token_budgets", torch.int32)
-    _, S, Hkv, D = cache_dims(kv_data, layout)
-    if Hkv != num_kv_heads:
-        raise ValueError("num_kv_heads does not match kv_data")
-    B, Hq, _ = q.shape
-    if o.shape != q.shape:
-        raise ValueError("o must have q's shape")
-    _lib.call("aoakv_decode_sparse_attn", q.data_ptr(), o.data_ptr(), kv_data.data_ptr(),
-              kv_indptr.data_ptr(), kv_indices.data_ptr(), kv_last_page_len.data_ptr(),
-              _ptr(sel_pages), 0 if sel_pages is None else sel_pages.shape[-1], token_budget,
-              _ptr(token_budgets), workspace.data_ptr(), workspace.numel(), B, max_pages, Hq,
-              Hkv, D, S, layout, flags, _stream())
+    _host.decode_sparse_attn(q, o, kv_data, kv_indptr, kv_indices, kv_last_page_len, sel_pages,
+                             token_budget, workspace, max_pages, num_kv_heads, layout,
+                             token_budgets, flags)
 
 
 def sparse_decode_layer(q, o, kv_data, kv_indptr, kv_indices, kv_last_page_len, metadata_data,
@@ -317,25 +208,10 @@ def sparse_decode_layer(q, o, kv_data, kv_indptr, kv_indices, kv_last_page_len, 
                         flags: int = FLAG_VALUE_AWARE | FLAG_FIXED, token_budgets=None):
     """Fused estimate + top-k + sparse decode for one layer (reference call
     sequence QuestAttention.py:135-157)."""
-    _need(q, "q", torch.float16)
-    _need(o, "o", torch.float16)
-    _need(kv_data, "kv_data", torch.float16)
-    _need(metadata_data, "metadata_data", torch.float16)
-    _need(scores, "scores", torch.float32)
-    _need(sel_pages, "sel_pages", torch.int32)
-    _need(workspace, "workspace", torch.uint8)
-    if flags & FLAG_VALUE_AWARE:
-        _need(v_log_norm, "v_log_norm", torch.float16)
-    if token_budgets is not None:
-        _need(token_budgets, "token_budgets", torch.int32)
-    _, S, Hkv, D = cache_dims(kv_data, layout)
-    B, Hq, _ = q.shape
-    _lib.call("aoakv_sparse_decode_layer", q.data_ptr(), o.data_ptr(), kv_data.data_ptr(),
-              kv_indptr.data_ptr(), kv_indices.data_ptr(), kv_last_page_len.data_ptr(),
-              metadata_data.data_ptr(), metadata_indptr.data_ptr(), metadata_indices.data_ptr(),
-              _ptr(v_log_norm), scores.data_ptr(), scores.shape[-1], sel_pages.data_ptr(),
-              sel_pages.shape[-1], token_budget, _ptr(token_budgets), workspace.data_ptr(),
-              workspace.numel(), B, max_pages, Hq, Hkv, D, S, layout, flags, _stream())
+    _host.sparse_decode_layer(q, o, kv_data, kv_indptr, kv_indices, kv_last_page_len,
+                              metadata_data, metadata_indptr, metadata_indices, v_log_norm,
+                              scores, sel_pages, token_budget, workspace, max_pages, layout,
+                              flags, token_budgets)
 
 
 def sparse_decode_layer_noalloc(q, o, kv_data, kv_indptr, kv_indices, kv_last_page_len,
@@ -407,19 +283,5 @@ def prefill_with_paged_kv_cache(q, kv_data, kv_indices, num_kv_pages: int, kv_la
                                 layout: int, causal: bool = True, o=None):
     """Reference: quest/ops/csrc/batch_prefill.cu:27-117.  q [L, Hq, D] -> o;
     the cache holds Hkv heads, Hq a multiple of Hkv (GQA)."""
-    _need(q, "q", torch.float16)
-    _need(kv_data, "kv_data", torch.float16)
-    _need(kv_indices, "kv_indices", torch.int32)
-    _, S, H, D = cache_dims(kv_data, layout)
-    if q.dim() != 3 or q.shape[2] != D:
-        raise ValueError(f"q must be [L, Hq, {D}], got {tuple(q.shape)}")
-    if o is None:
-        o = torch.empty_like(q)
-    n = _lib.load().aoakv_prefill_workspace_size(num_kv_pages, kv_last_page_len, q.shape[0],
-                                                 int(causal), q.shape[1], D, S)
-    # split keys: the chunks' partials, from torch's pool on this stream
-    ws = torch.empty(n, dtype=torch.uint8, device=q.device) if n else None
-    _lib.call("aoakv_prefill_with_workspace", q.data_ptr(), o.data_ptr(), kv_data.data_ptr(),
-              kv_indices.data_ptr(), num_kv_pages, kv_last_page_len, q.shape[0], int(causal),
-              q.shape[1], H, D, S, layout, _ptr(ws), n, _stream())
-    return o
+    return _host.prefill_with_paged_kv_cache(q, o, kv_data, kv_indices, num_kv_pages,
+                                             kv_last_page_len, layout, int(causal))

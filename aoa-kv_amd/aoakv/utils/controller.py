@@ -243,8 +243,26 @@ class InferenceController:
         self.metadata_cache.release()
         self._up.update(kv=0, md=0)
 
+    # the statistics of every layer, and a view per layer (made when they are
+    # set: every call of a layer takes its own)
+    @property
+    def v_log_norm(self) -> torch.Tensor:
+        return self._v_log_norm
+
+    @v_log_norm.setter
+    def v_log_norm(self, t: torch.Tensor):
+        self._v_log_norm, self._v_log_norm_layers = t, t.unbind(0)
+
+    @property
+    def v_mean(self) -> torch.Tensor:
+        return self._v_mean
+
+    @v_mean.setter
+    def v_mean(self, t: torch.Tensor):
+        self._v_mean, self._v_mean_layers = t, t.unbind(0)
+
     def v_log_norm_layer(self, layer_idx: int):
-        return self.v_log_norm[layer_idx]
+        return self._v_log_norm_layers[layer_idx]
 
     def v_mean_layer(self, layer_idx: int):
-        return self.v_mean[layer_idx]
+        return self._v_mean_layers[layer_idx]

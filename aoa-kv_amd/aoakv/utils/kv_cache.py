@@ -27,6 +27,8 @@ class KvPool:
         else:
             shape = (num_layers, capacity, 2, num_heads, block_len, head_dim)
         self._buf = torch.empty(shape, dtype=dtype, device=device)
+        # a view per layer, made once: every call of a layer takes its buffer
+        self._layers = self._buf.unbind(0)
         # free list; handed out lowest-first (or in a seeded random order, to
         # exercise non-identity page tables)
         free = list(range(capacity))
@@ -41,6 +43,10 @@ class KvPool:
     @property
     def buf(self):
         return self._buf
+
+    def layer(self, layer_idx: int):
+        assert layer_idx < len(self._layers)
+        return self._layers[layer_idx]
 
     @property
     def num_layers(self):
@@ -100,20 +106,19 @@ class KvCache:
         return self._indicies
 
     def buf_layer(self, layer_idx: int):
-        assert layer_idx < self.pool.num_layers
-        return self._pool.buf[layer_idx]
+        return self._pool.layer(layer_idx)
 
     def append_seq(self, seq_len: int) -> int:
         """Reserve space for tokens; return the number of new pages."""
         if seq_len <= 0:
             return 0
-        new = 0
-        for _ in range(seq_len):
-            if self._seqlen == 0 or self.last_page_len == self._pool.block_len:
-                self._indicies.append(self._pool.alloc_block())
-                new += 1
-            self._seqlen += 1
-        return new
+        page, had, total = self._pool.block_len, len(self._indicies), self._seqlen + seq_len
+        while len(self._indicies) * page < total:
+            # (the pages so far are full, also where the pool has no more)
+            self._seqlen = len(self._indicies) * page
+            self._indicies.append(self._pool.alloc_block())
+        self._seqlen = total
+        return len(self._indicies) - had
 
     def release(self):
         self._seqlen = 0

@@ -16,11 +16,22 @@
 
 namespace aoakv {
 RopeFreqs rope_freqs(float rope_scale, float rope_theta, uint32_t head_dim) {
+  // a program uses one set of factors: the last one's 32 to 128 powers are kept
+  thread_local struct {
+    float scale, theta;
+    uint32_t dim = 0u;
+    RopeFreqs r;
+  } last;
+  if (last.dim == head_dim && last.scale == rope_scale && last.theta == rope_theta) return last.r;
   RopeFreqs r{};
   const float rcp_scale = 1.0f / rope_scale, rcp_theta = 1.0f / rope_theta;
   for (uint32_t i = 0; i < head_dim / 2u; ++i)
     r.f[i] = (float)((double)rcp_scale *
                      std::pow((double)rcp_theta, (double)(2u * i) / (double)head_dim));
+  last.scale = rope_scale;
+  last.theta = rope_theta;
+  last.dim = head_dim;
+  last.r = r;
   return r;
 }
 }  // namespace aoakv
