@@ -29,7 +29,7 @@ HOST_LIB = os.path.join(PKG_DIR, "_host.so")
 HOST_SOURCE = "host.cpp"
 # build record beside the library (travels with it; the GPU box has no .git)
 BUILDINFO = os.path.join(PKG_DIR, "libaoakv.buildinfo.json")
-SOURCES = ["append.hip", "decode.hip", "prefill.hip", "generic.hip", "norm.hip", "capi.cpp"]
+SOURCES = ["append.hip", "decode.hip", "prefill.hip", "generic.hip", "stream.hip", "norm.hip", "capi.cpp"]
 REPO_DIR = os.path.dirname(os.path.dirname(PKG_DIR))
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

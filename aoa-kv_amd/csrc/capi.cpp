@@ -723,9 +723,10 @@ int aoakv_decode_sparse_attn(const void* q, void* o, const void* kv_data,
                           head_dim, page_size, layout, flags))
     return e;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return hip_status(aoakv::tuned_shape(head_dim, page_size)
+  return hip_status(aoakv::tuned_shape(head_dim, page_size) &&
+                            (sel_pages != nullptr || !aoakv::stream_dense(a, batch_size))
                         ? aoakv::launch_decode(a, batch_size, s)
-                        : aoakv::launch_gen_decode(a, batch_size, head_dim, s),
+                        : aoakv::launch_stream_decode(a, batch_size, head_dim, s),
                     "decode_sparse_attn");
 }
 
@@ -859,7 +860,7 @@ int aoakv_sparse_decode_layer(const void* q, void* o, const void* kv_data,
                                    batch_size, max_pages, head_dim, page_size, flags, s))
     return e;
   return hip_status(tuned ? aoakv::launch_decode(da, batch_size, s)
-                          : aoakv::launch_gen_decode(da, batch_size, head_dim, s),
+                          : aoakv::launch_stream_decode(da, batch_size, head_dim, s),
                     "sparse_decode_layer/decode");
 }
 

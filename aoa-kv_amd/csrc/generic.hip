@@ -10,15 +10,12 @@
 //     reductions inside a group are butterflies of wave shuffles;
 //   * page scores: one lane group per page, then the existing top-k kernel
 //     (which takes any page size);
-//   * decode: split over chunks of kGenChunkPages selected pages, one
-//     workgroup per (chunk, query head, sequence), online softmax per lane
-//     group, merged in LDS, then across chunks by the last to arrive;
+//   * decode: stream.hip;
 //   * prefill: one lane group per query, keys in order with an online
 //     softmax, no MFMA (the tuned MFMA kernel covers (128, 16)).
 // Arithmetic follows the tuned kernels where they define the reference's
 // rounding (fp16 filters, the fp32 page mean with one rounding, the fp16
-// running mean, the sequential fp32 norm of the log-norm, fp16 logits
-// rounded before and after the 1/sqrt(d) division).
+// running mean, the sequential fp32 norm of the log-norm).
 #include "kernels.hpp"
 
 namespace aoakv {
@@ -355,185 +352,6 @@ __global__ __launch_bounds__(256) void gen_estimate_kernel(EstimateArgs a) {
   }
 }
 
-// ---------------------------------------------------------------- decode
-// Attention of query head hq of sequence b over its selected pages (or all
-// of them), split over chunks of kGenChunkPages entries: one workgroup per
-// (chunk, query head, sequence) of W waves; wave w takes the chunk's entries
-// w, w + W, ..., lane group v of a wave the page's tokens v, v + 64/N, ...
-// W = 8 (a page per wave) when the grid has no more workgroups than the GPU
-// has CUs, else 4 (fewer registers per workgroup, more of them resident).
-// Logits fp16(q.k), then fp16(. / sqrt(d)) (quest_attention.py:265-268); online
-// softmax in fp32; the groups' (m, l, o) merged in LDS into the chunk's
-// partial.  A head of one chunk writes its output directly; otherwise the
-// last chunk to arrive at the head's counter merges the partials in chunk
-// order (the same arithmetic whichever workgroup merges) and clears them.
-// The quest_kernel convention attends the last page after the nsel selected
-// ones.
-// STREAM: no GQA group shares the pages' K/V, which are then loaded
-// non-temporally (as in the tuned decode)
-template <int D, uint32_t W, bool STREAM>
-__global__ __launch_bounds__(W * 64) void gen_decode_kernel(DecodeArgs a) {
-  static_assert(W == 4u || W == 8u, "4 or 8 waves");
-  constexpr uint32_t N = D / 8, GPW = kWave / N, G = W * GPW;  // groups per wave / block
-  constexpr uint32_t kStride = (uint32_t)D + 4u;                // partial: o[D], m, l, pad
-  __shared__ float s_o[G][D];
-  __shared__ float s_ml[G][2];
-  __shared__ uint32_t s_last;
-  const uint32_t l = threadIdx.x % N, grp = threadIdx.x / N;
-  const uint32_t wave = threadIdx.x / kWave, v = grp % GPW;
-  const uint32_t chunk = blockIdx.x, hq = blockIdx.y, b = blockIdx.z;
-  const uint32_t hkv = hq / (a.Hq / a.Hkv);
-  const bool quest = (a.flags & kFlagQuestKernel) != 0u;
-  const uint32_t S = a.S;
-  const uint32_t pbeg = (uint32_t)a.kv_indptr[b];
-  const uint32_t P_table = (uint32_t)a.kv_indptr[b + 1] - pbeg;
-  const uint32_t P = P_table < a.max_pages ? P_table : a.max_pages;
-  if (P != P_table && chunk == 0u && threadIdx.x == 0u) flag_error(a.error, kErrTruncated);
-  const uint32_t lpl = (uint32_t)a.kv_last_page_len[b];
-  if (P == 0u || lpl == 0u || lpl > S) return;  // malformed page table
-  const uint32_t budget = a.token_budgets ? (uint32_t)a.token_budgets[b] : a.token_budget;
-  uint32_t npages = P;
-  if (a.sel != nullptr) {
-    npages = num_selected_pages((P - 1u) * S + lpl, budget, S, P, quest ? kFlagQuestKernel : 0u);
-    const uint32_t row_cap = a.sel_stride + (quest ? 1u : 0u);
-    if (npages > row_cap) npages = row_cap;
-  }
-  // the grid holds max_chunks chunks per head: never index partials past it
-  if (npages > a.max_chunks * kGenChunkPages) {
-    npages = a.max_chunks * kGenChunkPages;
-    if (chunk == 0u && threadIdx.x == 0u) flag_error(a.error, kErrTruncated);
-  }
-  const uint32_t nch = (npages + kGenChunkPages - 1u) / kGenChunkPages;
-  if (chunk >= nch) return;  // uniform per block
-  const uint32_t nsel = (quest && a.sel != nullptr) ? npages - 1u : npages;
-  const int32_t* sel_row = a.sel ? a.sel + ((size_t)b * a.Hkv + hkv) * a.sel_stride : nullptr;
-  const uint32_t last_phys = (uint32_t)a.kv_indices[pbeg + P - 1u];
-  const H8 q = ld16(a.q + ((size_t)b * a.Hq + hq) * D + l * kVec);
-
-  float m = -INFINITY, lsum = 0.f, o[kVec];
-#pragma unroll
-  for (int j = 0; j < kVec; ++j) o[j] = 0.f;
-  const uint32_t ib = chunk * kGenChunkPages;  // the chunk's first entry (< npages)
-  const uint32_t i1 = ib + kGenChunkPages < npages ? ib + kGenChunkPages : npages;
-  // The wave's pages, entries ib + wave, ib + wave + W, ..., and their token
-  // counts (0: no page).  Group v takes tokens v, v + GPW, ... of each.  The
-  // K/V loads go out in batches of kB (page, token) slots, all of a batch
-  // before any is used (unconditional loads of clamped addresses: a slot
-  // past its page's tokens reads the page's slot 0, a missing page the
-  // chunk's first), so a wave waits on memory once per batch instead of
-  // once per token slot; the arithmetic runs in the same order as token by
-  // token.
-  constexpr uint32_t kPPW = kGenChunkPages / W;              // pages per wave
-  constexpr uint32_t kTPG = (kMaxPageSize + GPW - 1u) / GPW;  // token slots of a group per page
-  constexpr uint32_t kF = kPPW * kTPG;                        // ... over the wave's pages
-  constexpr uint32_t kB = kF < 8u ? kF : 8u;                  // slots loaded together
-  uint32_t ph[kPPW], nt[kPPW];
-#pragma unroll
-  for (uint32_t k = 0; k < kPPW; ++k) {
-    const uint32_t i = ib + wave + W * k;
-    const uint32_t ic = i < i1 ? i : ib;
-    uint32_t phys;
-    if (a.sel == nullptr) phys = (uint32_t)a.kv_indices[pbeg + ic];
-    else phys = ic < nsel ? (uint32_t)sel_row[ic] : last_phys;
-    ph[k] = phys;
-    nt[k] = i < i1 ? (phys == last_phys ? lpl : S) : 0u;
-  }
-  for (uint32_t f0 = 0; f0 < kF; f0 += kB) {
-    H8 kk[kB], vv[kB];
-#pragma unroll
-    for (uint32_t u = 0; u < kB; ++u) {
-      const uint32_t f = f0 + u, k = f / kTPG, j = f % kTPG;
-      if (GPW * j >= S) continue;  // uniform: slots past the page size
-      const uint32_t t = v + GPW * j;
-      const uint32_t tc = t < nt[k] ? t : 0u;
-      const f16* kp = a.kv + elem_off(a.g, ph[k], 0, hkv, tc) + l * kVec;
-      const f16* vp = a.kv + elem_off(a.g, ph[k], 1, hkv, tc) + l * kVec;
-      kk[u] = STREAM ? ld16_nt(kp) : ld16(kp);
-      vv[u] = STREAM ? ld16_nt(vp) : ld16(vp);
-    }
-#pragma unroll
-    for (uint32_t u = 0; u < kB; ++u) {
-      const uint32_t f = f0 + u, k = f / kTPG, j = f % kTPG;
-      const uint32_t t = v + GPW * j;
-      if (GPW * j >= S || t >= nt[k]) continue;  // (whole lane groups)
-      float acc = 0.f;
-#pragma unroll
-      for (int jj = 0; jj < kVec; ++jj) acc = acc + (float)q.v[jj] * (float)kk[u].v[jj];
-      const float x = (float)r16((float)r16(grp_sum_dpp<N>(acc)) / sqrt_d<D>());
-      const float mn = fmaxf(m, x);
-      const float c = m == -INFINITY ? 0.f : __expf(m - mn);
-      const float p = __expf(x - mn);
-      lsum = lsum * c + p;
-#pragma unroll
-      for (int jj = 0; jj < kVec; ++jj) o[jj] = o[jj] * c + p * (float)vv[u].v[jj];
-      m = mn;
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < kVec; ++j) s_o[grp][l * kVec + j] = o[j];
-  if (l == 0u) {
-    s_ml[grp][0] = m;
-    s_ml[grp][1] = lsum;
-  }
-  __syncthreads();
-  const size_t bh = (size_t)b * a.Hq + hq;
-  const uint32_t d = threadIdx.x;
-  if (d < (uint32_t)D) {
-    float M = -INFINITY;
-    for (uint32_t g2 = 0; g2 < G; ++g2) M = fmaxf(M, s_ml[g2][0]);
-    float acc = 0.f, Ls = 0.f;
-    for (uint32_t g2 = 0; g2 < G; ++g2) {
-      const float w = s_ml[g2][0] == -INFINITY ? 0.f : __expf(s_ml[g2][0] - M);
-      acc = acc + w * s_o[g2][d];
-      Ls = Ls + w * s_ml[g2][1];
-    }
-    if (nch == 1u) {
-      a.o[bh * D + d] = r16(acc / Ls);
-    } else {
-      float* part = a.partial + (bh * a.max_chunks + chunk) * kStride;
-      st_agent(part + d, acc);
-      if (d == 0u) {
-        st_agent(part + D, M);
-        st_agent(part + D + 1u, Ls);
-      }
-    }
-  }
-  if (nch == 1u) return;
-  if (!arrive_last(&a.counters[bh * kCounterStride], nch, &s_last)) return;
-  // the last chunk to arrive: merge every chunk's partial in chunk order,
-  // then clear the partials (the whole workspace stays zero between calls)
-  if (d < (uint32_t)D) {
-    // in groups of 16 chunks, every load of a group issued before any is
-    // used (one memory round trip per group), folded in chunk order
-    const float* base = a.partial + bh * a.max_chunks * kStride;
-    float M = -INFINITY, Ls = 0.f, acc = 0.f;
-    for (uint32_t c0 = 0; c0 < nch; c0 += 16u) {
-      float mc[16], lc[16], oc[16];
-#pragma unroll
-      for (uint32_t u = 0; u < 16u; ++u) {
-        const float* part = base + (c0 + u < nch ? c0 + u : nch - 1u) * kStride;
-        mc[u] = ld_agent(part + D);
-        lc[u] = ld_agent(part + D + 1u);
-        oc[u] = ld_agent(part + d);
-      }
-#pragma unroll
-      for (uint32_t u = 0; u < 16u; ++u) {
-        if (c0 + u >= nch) break;  // uniform
-        const float Mn = fmaxf(M, mc[u]);
-        const float keep = M == -INFINITY ? 0.f : __expf(M - Mn);
-        const float w = mc[u] == -INFINITY ? 0.f : __expf(mc[u] - Mn);
-        Ls = Ls * keep + w * lc[u];
-        acc = acc * keep + w * oc[u];
-        M = Mn;
-      }
-    }
-    a.o[bh * D + d] = r16(acc / Ls);
-  }
-  __syncthreads();  // every thread has read the partials
-  uint32_t* pw = reinterpret_cast<uint32_t*>(a.partial + bh * a.max_chunks * kStride);
-  for (uint32_t i = threadIdx.x; i < nch * kStride; i += W * 64u) st_agent_u32(pw + i, 0u);
-}
-
 // ---------------------------------------------------------------- prefill
 // Causal (or full) attention of Lq queries, the last Lq positions of an
 // L-token paged sequence: one lane group per (query, head), keys in order,
@@ -656,31 +474,6 @@ hipError_t launch_gen_estimate(const EstimateArgs& a, uint32_t batch, uint32_t m
       case 8: hipLaunchKernelGGL((gen_estimate_kernel<D, 8>), grid, dim3(256), 0, s, a); break;
       default: return hipErrorInvalidValue;
     }
-  })
-  return hipGetLastError();
-}
-
-hipError_t launch_gen_decode(const DecodeArgs& a, uint32_t batch, uint32_t D_, hipStream_t s) {
-  // 8 waves (a page each) while the grid fits the GPU's 256 CUs once over
-  // (32k context, budget 2048: head dim 256 19.9 -> 15.2 us, page size 32
-  // 18.4 -> 14.4); with more workgroups, 4 waves, of which more fit per CU
-  // (page size 8, 1,024 workgroups: 15.5 us with 4 waves, 30.9 with 8).
-  // Without GQA the K/V loads stream (non-temporal): over 32 rotated layers
-  // head dim 64 23.1 -> 22.2 us per layer (scores + decode), 256 34.4 ->
-  // 32.5, page size 8 41.4 -> 39.1, page size 32 27.9 -> 27.0, with the
-  // scoring's metadata streamed too
-  const bool wide = (size_t)a.max_chunks * a.Hq * batch <= 256u;
-  const bool stream = a.Hq == a.Hkv;
-  const dim3 grid(a.max_chunks, a.Hq, batch);
-  AOAKV_GEN_D(D_, {
-    if (wide && stream)
-      hipLaunchKernelGGL((gen_decode_kernel<D, 8, true>), grid, dim3(512), 0, s, a);
-    else if (wide)
-      hipLaunchKernelGGL((gen_decode_kernel<D, 8, false>), grid, dim3(512), 0, s, a);
-    else if (stream)
-      hipLaunchKernelGGL((gen_decode_kernel<D, 4, true>), grid, dim3(256), 0, s, a);
-    else
-      hipLaunchKernelGGL((gen_decode_kernel<D, 4, false>), grid, dim3(256), 0, s, a);
   })
   return hipGetLastError();
 }

@@ -27,13 +27,13 @@ __device__ inline void flag_error(uint32_t* error, uint32_t bits) {
   if (error != nullptr) atomicOr(error, bits);
 }
 
-// Selected pages per decode chunk of the generic kernels (as the tuned
-// kernels' 8): the workspace's partials are laid out per chunk of 8.
+// Pages per decode chunk of stream.hip at least (as the tuned kernels' 8):
+// the workspace's partials are laid out per chunk of 8.
 constexpr uint32_t kGenChunkPages = 8u;
 
 // Head dims the library takes: the tuned kernels are for kHeadDim (with
 // kPageSize); 64 and 256, and other page sizes up to kMaxPageSize, run the
-// kernels of generic.hip.
+// kernels of generic.hip and stream.hip.
 constexpr int kMaxHeadDim = 256;
 constexpr uint32_t kMaxPageSize = 32;
 inline bool tuned_shape(uint32_t head_dim, uint32_t page_size) {
@@ -256,6 +256,12 @@ uint32_t layer_stagger_ps(uint32_t est_chunks, uint32_t group, uint32_t heads); 
 uint32_t counter_stride();        // u32 words between per-head counters (one cache line each)
 uint32_t layer_self_blocks_per_cu(uint32_t group, uint32_t heads_per_item, uint32_t score_heads);  // per CU
 
+// stream.hip: dense decode (a.sel == nullptr, any shape), and the selected
+// pages of the shapes without tuned kernels
+bool stream_dense(const DecodeArgs& a, uint32_t batch);  // the tuned shape's, else decode.hip
+hipError_t launch_stream_decode(const DecodeArgs& a, uint32_t batch, uint32_t head_dim,
+                                hipStream_t s);
+
 // generic.hip: the other head dims (64, 128, 256) and page sizes (1..32)
 hipError_t launch_gen_append_prefill(const AppendPrefillArgs& a, uint32_t head_dim, hipStream_t s);
 hipError_t launch_gen_append_decode(const AppendDecodeArgs& a, uint32_t batch, uint32_t head_dim,
@@ -263,8 +269,6 @@ hipError_t launch_gen_append_decode(const AppendDecodeArgs& a, uint32_t batch, u
 hipError_t launch_gen_rope(const RopeArgs& a, uint32_t head_dim, hipStream_t s);
 hipError_t launch_gen_estimate(const EstimateArgs& a, uint32_t batch, uint32_t max_pages,
                                uint32_t head_dim, hipStream_t s);
-hipError_t launch_gen_decode(const DecodeArgs& a, uint32_t batch, uint32_t head_dim,
-                             hipStream_t s);
 hipError_t launch_gen_prefill(const PrefillArgs& a, uint32_t head_dim, hipStream_t s);
 
 }  // namespace aoakv

@@ -365,3 +365,36 @@ def test_unsupported_shapes_are_refused():
         with pytest.raises(RuntimeError, match="unsupported"):
             append_kv(k, k, c, 0)
     assert _lib.load() is not None
+
+
+# (D, S, heads, kv heads, layout, tokens): a stream of each group size (1, 2,
+# 4, 8), a partial last page, a chunk whose page ids are staged twice (256
+# heads of 550 one-token pages each), a page size that does not divide a
+# batch, fewer tokens than one batch, one token
+STREAM = [(128, 16, 32, 32, HND, 4101), (256, 16, 16, 8, NHD, 8200), (128, 16, 32, 8, NHD, 8299),
+          (64, 3, 64, 8, HND, 1550), (64, 1, 256, 256, HND, 1100), (256, 7, 8, 8, HND, 1000),
+          (128, 32, 4, 4, NHD, 33), (64, 16, 8, 2, HND, 5), (256, 1, 2, 2, HND, 1)]
+
+
+@pytest.mark.parametrize("D,S,H,hkv,layout,L", STREAM)
+def test_dense_decode_streams(D, S, H, hkv, layout, L):
+    """decode_sparse_attn over every page against the simulation's dense decode,
+    twice (the partials are cleared); the cache's unwritten slots are NaN."""
+    from aoakv.utils import append_kv, decode_sparse_attn
+    _say(f"[dense stream] D={D} S={S} heads={H}/{hkv} layout={layout} L={L}")
+    c = _ctrl(H, D, S, L + 2 * S, layout, 4 * S, hkv=hkv)
+    c.kv_cache.buf_layer(0).fill_(float("nan"))
+    c.prepare_metadata(L)
+    c.begin_forward(L)
+    K, V = randn16(L, (L, hkv, D)), randn16(L + 1, (L, hkv, D))
+    k, v = torch.from_numpy(K).to(DEV), torch.from_numpy(V).to(DEV)
+    append_kv(k, v, c, 0)
+    c.begin_forward(1)
+    q = randn16(L + 2, (1, H, D))
+    qd = torch.from_numpy(q).to(DEV)
+    o = [decode_sparse_attn(qd, c, 0, None).cpu().numpy() for _ in range(2)]
+    assert np.array_equal(bits(o[0]), bits(o[1]))
+    rep = lambda x: np.repeat(x.transpose(1, 0, 2), H // hkv, 0)[None]
+    ref = sim.masked_decode_attention(q.transpose(1, 0, 2)[None], rep(K), rep(V), None)[0, :, 0]
+    assert np.abs(o[0][0].astype(np.float32) - ref.astype(np.float32)).max() <= 2e-3
+    assert int(c.workspace[64 * 4:].count_nonzero()) == 0  # all of it zero again
