@@ -838,7 +838,9 @@ int aoakv_sparse_decode_layer(const void* q, void* o, const void* kv_data,
     if (la.self_select) la.e.hscore_copies = copies;
     return hip_status(aoakv::launch_layer(la, s), "sparse_decode_layer");
   }
-  if (tuned && max_pages <= aoakv::fused_topk_max_pages()) {
+  const bool selects = tuned ? max_pages <= aoakv::fused_topk_max_pages()
+                             : aoakv::stream_selects(da, batch_size, max_pages);
+  if (selects) {
     // two launches: the scores alone (the unfused kernel, smaller items),
     // then decode items that each select their kv head's pages from the
     // complete scores (16 copies of every top-k, none waiting on another
@@ -847,14 +849,19 @@ int aoakv_sparse_decode_layer(const void* q, void* o, const void* kv_data,
     // the scoring launch's last item per head (13.0 + 11.1); before the
     // streamed loads 24.7-25.1 against 25.6, and starting the kv heads'
     // decode items 0.1-0.3 us apart was slower (25.1-30.0).
-    if (int e = hip_status(aoakv::launch_estimate(ea, batch_size, max_pages, s), "estimate"))
+    if (int e = hip_status(
+            tuned ? aoakv::launch_estimate(ea, batch_size, max_pages, s)
+                  : aoakv::launch_gen_estimate(ea, batch_size, max_pages, head_dim, s),
+            "estimate"))
       return e;
     aoakv::EstimateArgs es = ea;
     es.sel = sel_pages;
     es.sel_stride = sel_stride;
     es.token_budget = token_budget;
     es.token_budgets = token_budgets;
-    return hip_status(aoakv::launch_decode(da, batch_size, s, &es), "sparse_decode_layer/decode");
+    return hip_status(tuned ? aoakv::launch_decode(da, batch_size, s, &es)
+                            : aoakv::launch_stream_decode(da, batch_size, head_dim, s, &es),
+                      "sparse_decode_layer/decode");
   }
   if (int e = launch_estimate_topk(ea, w, sel_pages, sel_stride, token_budget, token_budgets,
                                    batch_size, max_pages, head_dim, page_size, flags, s))

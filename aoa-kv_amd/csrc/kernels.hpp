@@ -259,8 +259,11 @@ uint32_t layer_self_blocks_per_cu(uint32_t group, uint32_t heads_per_item, uint3
 // stream.hip: dense decode (a.sel == nullptr, any shape), and the selected
 // pages of the shapes without tuned kernels
 bool stream_dense(const DecodeArgs& a, uint32_t batch);  // the tuned shape's, else decode.hip
+// self: the decode selects for itself, as launch_decode's (where stream_selects
+// says so)
+bool stream_selects(const DecodeArgs& a, uint32_t batch, uint32_t max_pages);
 hipError_t launch_stream_decode(const DecodeArgs& a, uint32_t batch, uint32_t head_dim,
-                                hipStream_t s);
+                                hipStream_t s, const EstimateArgs* self = nullptr);
 
 // generic.hip: the other head dims (64, 128, 256) and page sizes (1..32)
 hipError_t launch_gen_append_prefill(const AppendPrefillArgs& a, uint32_t head_dim, hipStream_t s);

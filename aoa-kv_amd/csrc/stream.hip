@@ -20,13 +20,15 @@
 // dim 64 at 20000 153 -> 63, 256 (16 heads) at 8000 95 -> 58; one selected
 // layer of 128 pages x 16 heads of dim 256 (decode alone) 16.2 -> 13.3.
 #include "kernels.hpp"
+#include "topk.hpp"
 
 namespace aoakv {
 namespace {
 
-constexpr uint32_t kStThreads = 256;
+constexpr uint32_t kStThreads = kThreads;
 constexpr uint32_t kStWaves = kStThreads / kWave;
 constexpr uint32_t kStListPages = 512;  // pages whose ids are staged at a time
+constexpr uint32_t kStSelfWorkgroups = 1024;  // 4 per CU (36 KB of LDS each)
 constexpr int kU = 4;                   // loads of K (and of V) per batch
 constexpr float kNoMax = -1e30f;        // running max before the first token: finite
 
@@ -92,6 +94,11 @@ __device__ inline float logit_f16(float x) {
 struct StreamArgs : DecodeArgs {
   uint32_t grid_chunks;
   uint32_t page_rcp;
+  // SELF: the rows the selection is made from (complete), and where it goes
+  const float* scores;
+  uint32_t score_stride;
+  uint32_t select_flags;
+  int32_t* sel_out;
 };
 
 // One workgroup per (chunk of the page list, G query heads of a kv head,
@@ -100,7 +107,10 @@ struct StreamArgs : DecodeArgs {
 // pages); the last to arrive at the head's counter merges their partials in
 // chunk order and clears them.
 // NT: no other workgroup reads these pages: non-temporal loads.
-template <int D, int G, bool NT>
+// SELF: there are no selection rows yet; every workgroup of a kv head runs the
+// head's top-k on the scores the previous launch wrote, takes its chunk's
+// entries and writes them out (as decode.hip's two-launch layer).
+template <int D, int G, bool NT, bool SELF = false>
 __global__ __launch_bounds__(kStThreads) void stream_decode_kernel(StreamArgs a) {
   constexpr uint32_t N = D / 8, GPW = kWave / N;  // lanes per group, groups per wave
   constexpr uint32_t kBatch = kU * GPW;           // tokens
@@ -109,10 +119,19 @@ __global__ __launch_bounds__(kStThreads) void stream_decode_kernel(StreamArgs a)
   // against 38.5 us, pages of 8 127.8 against 115.1 per 4 layers)
   constexpr int kAhead = 2;
   constexpr uint32_t kStride = (uint32_t)D + 4u;  // partial: o[D], m, l, pad
-  __shared__ uint32_t s_page[kStListPages];
-  __shared__ float s_o[kStWaves][G][D];
-  __shared__ float s_ml[kStWaves][G][2];
+  struct Shared {
+    float o[kStWaves][G][D];
+    float ml[kStWaves][G][2];
+  };
+  struct Empty {};
+  __shared__ uint32_t s_page[SELF ? kGenChunkPages : kStListPages];
+  __shared__ union {
+    typename std::conditional<SELF, TopkShared, Empty>::type tk;
+    Shared d;
+  } sm;
   __shared__ uint32_t s_last;
+  auto& s_o = sm.d.o;
+  auto& s_ml = sm.d.ml;
   const uint32_t lane = __lane_id();
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint32_t l = lane % N, v = lane / N;
@@ -162,15 +181,47 @@ __global__ __launch_bounds__(kStThreads) void stream_decode_kernel(StreamArgs a)
     for (int j = 0; j < kVec; ++j) o[g][j] = 0.f;
   }
   const uint32_t i0 = chunk * per, i1 = i0 + per < npages ? i0 + per : npages;
+  if constexpr (SELF) {
+    static_assert(G == 1, "a query head per workgroup");
+    // candidates: every scored page (quest_kernel: but the last); the
+    // selection's first nout entries, in page order
+    const uint32_t row = P < a.score_stride + (quest ? 1u : 0u) ? P
+                                                               : a.score_stride + (quest ? 1u : 0u);
+    const uint32_t cand = quest ? row - 1u : row;
+    uint32_t k = num_selected_pages((row - 1u) * S + lpl, budget, S, row, a.select_flags);
+    if (quest) k -= 1u;
+    if (k > a.sel_stride) k = a.sel_stride;
+    const int32_t* ids = a.kv_indices + pbeg;
+    const bool pick = k != 0u && k < cand;
+    if (pick)
+      topk_staged<true>(a.scores + ((size_t)b * a.Hkv + hkv) * a.score_stride, cand, k,
+                        (a.select_flags & kFlagFixed) != 0u, ids, nullptr, sm.tk);
+    const uint32_t nout = pick ? k : (k == 0u ? 0u : cand);
+    // this chunk's entries, here and in the selection output (whose end the
+    // last chunk writes); an entry the top-k did not yield means the shapes
+    // disagree
+    int32_t* out = a.sel_out + ((size_t)b * a.Hkv + hkv) * a.sel_stride;
+    auto entry = [&](uint32_t i) { return pick ? sm.tk.key[i] : (uint32_t)ids[i]; };
+    if (threadIdx.x < per) {  // per = kGenChunkPages
+      const uint32_t i = i0 + threadIdx.x;
+      if (i < nsel && i >= nout) flag_error(a.error, kErrTruncated);
+      s_page[threadIdx.x] = i >= nsel ? last_phys : i < nout ? entry(i) : last_phys;
+    }
+    const uint32_t o_end = chunk == nch - 1u || i0 + per > nout ? nout : i0 + per;
+    for (uint32_t i = i0 + threadIdx.x; i < o_end; i += kStThreads) out[i] = (int32_t)entry(i);
+    __syncthreads();  // (the top-k's memory is the softmax's from here)
+  }
   for (uint32_t ib = i0; ib < i1; ib += kStListPages) {
     // ---- the ids of up to kStListPages pages of the list
     const uint32_t np = i1 - ib < kStListPages ? i1 - ib : kStListPages;
-    if (ib != i0) __syncthreads();  // the ids before were read
-    for (uint32_t i = threadIdx.x; i < np; i += kStThreads)
-      s_page[i] = sel_row == nullptr ? (uint32_t)a.kv_indices[pbeg + ib + i]
-                  : ib + i < nsel    ? (uint32_t)sel_row[ib + i]
-                                     : last_phys;
-    __syncthreads();
+    if constexpr (!SELF) {
+      if (ib != i0) __syncthreads();  // the ids before were read
+      for (uint32_t i = threadIdx.x; i < np; i += kStThreads)
+        s_page[i] = sel_row == nullptr ? (uint32_t)a.kv_indices[pbeg + ib + i]
+                    : ib + i < nsel    ? (uint32_t)sel_row[ib + i]
+                                       : last_phys;
+      __syncthreads();
+    }
     const uint32_t T = np * S;  // token slots
     const uint32_t nb = (T + kBatch - 1u) / kBatch;
     // loads of batch i (clamped: a slot past the end reads the last one), and
@@ -332,6 +383,13 @@ __global__ __launch_bounds__(kStThreads) void stream_decode_kernel(StreamArgs a)
 template <int D>
 hipError_t launch_d(const StreamArgs& a, uint32_t G, dim3 grid, hipStream_t s) {
   const dim3 block(kStThreads);
+  if (a.scores != nullptr) {
+    if (a.Hq == a.Hkv)
+      hipLaunchKernelGGL((stream_decode_kernel<D, 1, true, true>), grid, block, 0, s, a);
+    else
+      hipLaunchKernelGGL((stream_decode_kernel<D, 1, false, true>), grid, block, 0, s, a);
+    return hipGetLastError();
+  }
   // K/V of one reader: no GQA group, or a whole group per workgroup
   if (G > 1u || a.Hq == a.Hkv) {
     switch (G) {
@@ -367,9 +425,26 @@ bool stream_dense(const DecodeArgs& a, uint32_t batch) {
          (a.Hq == a.Hkv && (uint64_t)a.max_chunks * a.Hq * batch >= 1024u);
 }
 
+// The layers whose decode selects for itself: rows the top-k stages, and no
+// more workgroups than are resident at once (each repeats its head's top-k,
+// which spares the launch of its own, 5.9 us).  Four layers: head dim 256,
+// 20011 tokens, 256 workgroups 118 -> 108 us; 64 x 32 heads, 32768 tokens, 512
+// workgroups 82 -> 75; with 2048 workgroups (pages of 8, budget 4096) 187 and
+// selecting for themselves 222.
+bool stream_selects(const DecodeArgs& a, uint32_t batch, uint32_t max_pages) {
+  return max_pages <= kStageMaxPages && (uint64_t)a.max_chunks * a.Hq * batch <= kStSelfWorkgroups;
+}
+
 hipError_t launch_stream_decode(const DecodeArgs& args, uint32_t batch, uint32_t head_dim,
-                                hipStream_t s) {
-  StreamArgs a{args, 0u, 0u};
+                                hipStream_t s, const EstimateArgs* self) {
+  StreamArgs a{};
+  static_cast<DecodeArgs&>(a) = args;
+  if (self != nullptr) {
+    a.scores = self->scores;
+    a.score_stride = self->score_stride;
+    a.select_flags = self->flags;
+    a.sel_out = self->sel;
+  }
   a.page_rcp = a.S > 1u ? (uint32_t)((1ull << 32) / a.S) + 1u : 0u;
   const bool dense = a.sel == nullptr;
   const uint32_t G = dense ? dense_group(a, batch) : 1u, heads = a.Hq / G;

@@ -398,3 +398,38 @@ def test_dense_decode_streams(D, S, H, hkv, layout, L):
     ref = sim.masked_decode_attention(q.transpose(1, 0, 2)[None], rep(K), rep(V), None)[0, :, 0]
     assert np.abs(o[0][0].astype(np.float32) - ref.astype(np.float32)).max() <= 2e-3
     assert int(c.workspace[64 * 4:].count_nonzero()) == 0  # all of it zero again
+
+
+# (D, S, heads, kv heads, tokens, budget, semantics): rows of exactly as many
+# pages as a workgroup stages and of one more (the top-k as a launch of its
+# own), more workgroups than are resident (the same), GQA, everything
+# selected, a one-page budget (nothing to select), a selection that ends
+# inside a chunk
+SELF = [(64, 1, 4, 4, 4096, 100, "sim"), (64, 1, 4, 2, 4097, 100, "sim"),
+        (128, 1, 64, 64, 700, 136, "sim"), (256, 16, 8, 4, 1000, 208, "sim"),
+        (64, 8, 8, 2, 900, 4096, "sim"), (256, 32, 4, 4, 1000, 32, "quest_kernel"),
+        (64, 16, 8, 1, 2000, 272, "quest_kernel"), (128, 7, 4, 4, 333, 77, "sim")]
+
+
+@pytest.mark.parametrize("D,S,H,hkv,L,budget,semantics", SELF)
+def test_layer_that_selects_in_its_decode_equals_the_three_calls(D, S, H, hkv, L, budget,
+                                                                 semantics):
+    from aoakv.utils import (InferenceController, decode_estimate, decode_layer,
+                             decode_sparse_attn, decode_topk)
+    _say(f"[self select] D={D} S={S} heads={H}/{hkv} L={L} budget={budget} {semantics}")
+    c = InferenceController(1, H, D, S, budget // S, L + S, torch.float16, DEV, num_kv_heads=hkv,
+                            shuffle_seed=3, semantics=semantics)
+    _prefill(c, randn16(L, (1, hkv, L, D)), randn16(L + 1, (1, hkv, L, D)))
+    c.begin_forward(1)
+    q = torch.from_numpy(randn16(L + 2, (1, H, D))).to(DEV)
+    scores = decode_estimate(q, c, 0).clone()
+    sel = decode_topk(scores, c).clone()
+    o = decode_sparse_attn(q, c, 0, c.topk_dindices_buffer)
+    for _ in range(2):
+        c._sel.fill_(-1)
+        c.scores.fill_(float("nan"))
+        o2 = decode_layer(q, c, 0)
+        assert torch.equal(o2, o)
+        assert torch.equal(c.topk_dindices_buffer[0], sel)
+        assert torch.equal(c.scores[0, :, :scores.shape[1]], scores)
+    c.check_errors()
