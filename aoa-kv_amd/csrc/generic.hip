@@ -254,16 +254,22 @@ __global__ __launch_bounds__(256) void gen_rope_kernel(RopeArgs a) {
 }
 
 // ---------------------------------------------------------------- page scores
-// Pages [64 x, 64 x + 64) of (sequence b, kv head h): one lane group per
-// page.  Score of a page (filter_util.py:269-330, as score_item): per query
-// head g of the group, x_g = sum_d max(q_d Kmax_d, q_d Kmin_d) (fp32); the
-// value-aware score is logsumexp_g(2 x_g / sqrt(d)) + 2 log-norm, plain
-// Quest sums x_g over the group.
-constexpr uint32_t kGenPagesPerBlock = 64;
+// Pages [n x, n x + n), n = gen_block_pages, of (sequence b, kv head h): one
+// lane group per page.  Score of a page (filter_util.py:269-330, as
+// score_item): per query head g of the group, x_g = sum_d max(q_d Kmax_d, q_d
+// Kmin_d) (fp32); the value-aware score is logsumexp_g(2 x_g / sqrt(d)) + 2
+// log-norm, plain Quest sums x_g over the group.
+// A page per lane group and no more: the page's arithmetic (a division, with
+// GQA an exponential per query head and a logarithm) is a serial chain, which
+// several pages per group made longer.  Four layers at 20011 tokens, head dim
+// 256: 64 pages per block 106 us, 32 101, 16 97, 8 (one per group) 95; with 16
+// / 8 heads 103, 90, 84, 79.
+template <int D>
+constexpr uint32_t gen_block_pages() { return 256u / (D / 8); }
 
 template <int D, int GROUP>
 __global__ __launch_bounds__(256) void gen_estimate_kernel(EstimateArgs a) {
-  constexpr uint32_t N = D / 8, PPS = 256u / N;  // pages per step of the block
+  constexpr uint32_t N = D / 8;
   const uint32_t l = threadIdx.x % N;
   const uint32_t b = blockIdx.z, h = blockIdx.y;
   const uint32_t pbeg = (uint32_t)a.kv_indptr[b];
@@ -281,75 +287,50 @@ __global__ __launch_bounds__(256) void gen_estimate_kernel(EstimateArgs a) {
 #pragma unroll
   for (int g = 0; g < GROUP; ++g)
     q[g] = ld16(a.q + ((size_t)b * a.Hq + h * GROUP + g) * D + l * kVec);
-  const uint32_t pb = blockIdx.x * kGenPagesPerBlock;  // the block's first page
-  if (pb >= nstore) return;                            // uniform
-  const uint32_t p_end = pb + kGenPagesPerBlock < nstore ? pb + kGenPagesPerBlock : nstore;
-  // The block's pages in kSt steps of PPS, group g taking page pb + g + s *
-  // PPS at step s.  Every step's page-table words are loaded together, then
-  // every step's metadata and value statistic (unconditional loads of
-  // clamped pages: a page past the block's end reads its first), so the
-  // block waits on two round trips, not two or three per step; the scores
-  // are computed in the same order as step by step.
-  constexpr uint32_t kSt = kGenPagesPerBlock / PPS;
-  uint32_t mpg[kSt], phys[kSt];
+  const uint32_t pb = blockIdx.x * gen_block_pages<D>();  // the block's first page
+  if (pb >= nstore) return;                               // uniform
+  // this group's page (unconditional loads: one past the end reads the
+  // block's first; it is not stored)
+  const uint32_t p = pb + threadIdx.x / N, pc = p < nstore ? p : pb;
+  const uint32_t mpg = (uint32_t)a.meta_indices[mbeg + pc / a.S];
+  const uint32_t phys = value_aware ? (uint32_t)a.kv_indices[pbeg + pc] : 0u;
+  const size_t off = elem_off(a.g, mpg, 0, h, pc % a.S) + l * kVec;
+  // read once: non-temporal loads, as the tuned scoring's
+  const H8 kmx = ld16_nt(a.meta + off), kmn = ld16_nt(a.meta + off + a.g.kv);
+  const f16 lvn = value_aware ? a.v_log_norm[(size_t)phys * a.Hkv + h] : (f16)0.f;
+  float x[GROUP];
 #pragma unroll
-  for (uint32_t st = 0; st < kSt; ++st) {
-    const uint32_t p = pb + threadIdx.x / N + st * PPS;
-    const uint32_t pc = p < p_end ? p : pb;
-    mpg[st] = (uint32_t)a.meta_indices[mbeg + pc / a.S];
-    phys[st] = value_aware ? (uint32_t)a.kv_indices[pbeg + pc] : 0u;
+  for (int g = 0; g < GROUP; ++g) {
+    float acc = 0.f;
+#pragma unroll
+    for (int j = 0; j < kVec; ++j) {
+      const float qv = (float)q[g].v[j];
+      acc = acc + fmaxf(qv * (float)kmx.v[j], qv * (float)kmn.v[j]);
+    }
+    x[g] = grp_sum_dpp<N>(acc);
   }
-  H8 kmxs[kSt], kmns[kSt];
-  f16 lvn[kSt];
-#pragma unroll
-  for (uint32_t st = 0; st < kSt; ++st) {
-    const uint32_t p = pb + threadIdx.x / N + st * PPS;
-    const uint32_t pc = p < p_end ? p : pb;
-    const size_t off = elem_off(a.g, mpg[st], 0, h, pc % a.S) + l * kVec;
-    // read once: non-temporal loads, as the tuned scoring's
-    kmxs[st] = ld16_nt(a.meta + off);
-    kmns[st] = ld16_nt(a.meta + off + a.g.kv);
-    lvn[st] = value_aware ? a.v_log_norm[(size_t)phys[st] * a.Hkv + h] : (f16)0.f;
-  }
-#pragma unroll
-  for (uint32_t st = 0; st < kSt; ++st) {
-    const uint32_t p = pb + threadIdx.x / N + st * PPS;
-    if (p >= p_end) break;  // (whole lane groups; later steps lie further on)
-    const H8 kmx = kmxs[st], kmn = kmns[st];
-    float x[GROUP];
+  float score;
+  if (value_aware) {
+    float m = -INFINITY;
 #pragma unroll
     for (int g = 0; g < GROUP; ++g) {
-      float acc = 0.f;
-#pragma unroll
-      for (int j = 0; j < kVec; ++j) {
-        const float qv = (float)q[g].v[j];
-        acc = acc + fmaxf(qv * (float)kmx.v[j], qv * (float)kmn.v[j]);
-      }
-      x[g] = grp_sum_dpp<N>(acc);
+      x[g] = 2.0f * (x[g] / sqrt_d<D>());
+      m = fmaxf(m, x[g]);
     }
-    float score;
-    if (value_aware) {
-      float m = -INFINITY;
+    score = x[0];
+    if (GROUP > 1) {
+      float se = 0.f;
 #pragma unroll
-      for (int g = 0; g < GROUP; ++g) {
-        x[g] = 2.0f * (x[g] / sqrt_d<D>());
-        m = fmaxf(m, x[g]);
-      }
-      score = x[0];
-      if (GROUP > 1) {
-        float se = 0.f;
-#pragma unroll
-        for (int g = 0; g < GROUP; ++g) se = se + expf(x[g] - m);
-        score = logf(se) + m;
-      }
-      score = score + 2.0f * (float)lvn[st];
-    } else {
-      score = x[0];
-#pragma unroll
-      for (int g = 1; g < GROUP; ++g) score = score + x[g];
+      for (int g = 0; g < GROUP; ++g) se = se + expf(x[g] - m);
+      score = logf(se) + m;
     }
-    if (l == 0u) a.scores[((size_t)b * a.Hkv + h) * a.score_stride + p] = score;
+    score = score + 2.0f * (float)lvn;
+  } else {
+    score = x[0];
+#pragma unroll
+    for (int g = 1; g < GROUP; ++g) score = score + x[g];
   }
+  if (l == 0u && p < nstore) a.scores[((size_t)b * a.Hkv + h) * a.score_stride + p] = score;
 }
 
 // ---------------------------------------------------------------- prefill
@@ -464,9 +445,9 @@ hipError_t launch_gen_rope(const RopeArgs& a, uint32_t D_, hipStream_t s) {
 
 hipError_t launch_gen_estimate(const EstimateArgs& a, uint32_t batch, uint32_t max_pages,
                                uint32_t D_, hipStream_t s) {
-  const dim3 grid((max_pages + kGenPagesPerBlock - 1) / kGenPagesPerBlock, a.Hkv, batch);
   const uint32_t group = a.Hq / a.Hkv;
   AOAKV_GEN_D(D_, {
+    const dim3 grid((max_pages + gen_block_pages<D>() - 1) / gen_block_pages<D>(), a.Hkv, batch);
     switch (group) {
       case 1: hipLaunchKernelGGL((gen_estimate_kernel<D, 1>), grid, dim3(256), 0, s, a); break;
       case 2: hipLaunchKernelGGL((gen_estimate_kernel<D, 2>), grid, dim3(256), 0, s, a); break;
