@@ -47,6 +47,11 @@ constexpr uint32_t est_kernel_block_pages() {
 __host__ __device__ constexpr uint32_t est_kernel_block_pages_of(uint32_t group, bool fused) {
   return group == 1u && !fused ? est_block_pages_of(1u) / 2u : est_block_pages_of(group);
 }
+// ... and a page per 16-lane row where those would leave CUs without one:
+// estimate, top-k and attention at 32 heads, 4096 tokens (128 items of 64
+// pages) 17.3 -> 16.8 us, 8192 (256) 17.7 -> 17.5; but 16384 (512) 18.0 -> 18.5.
+constexpr uint32_t kEstSmallPages = 16;
+constexpr uint64_t kEstSmallItems = 256;
 constexpr int kDecPagesPerWave = 2;
 constexpr int kDecPagesPerBlock = kDecPagesPerWave * 4;  // 8
 constexpr int kPartialStride = kHeadDim + 4;             // o[128], m, l, pad
@@ -370,13 +375,12 @@ __device__ __forceinline__ void select_item(const EstimateArgs& a, uint32_t b, u
 
 // Scores one chunk; with a.sel set, the last block of the head to finish
 // also selects its pages (arrival counter per head).
-template <int GROUP, bool FUSED>
+template <int GROUP, bool FUSED, uint32_t kPPB = est_kernel_block_pages<GROUP, FUSED>()>
 __device__ __forceinline__ void estimate_item(const EstimateArgs& a, uint32_t b, uint32_t h,
                                               uint32_t chunk, EstShared& sm, TopkShared* tk) {
   // the fused top-k's shape, loaded up front (off the handoff path)
   SelPlan plan{};
   if (a.sel != nullptr) plan = plan_select(a, b);
-  constexpr uint32_t kPPB = est_kernel_block_pages<GROUP, FUSED>();
   if (!score_item<GROUP, kPPB>(a, b, h, chunk, sm)) return;
   if (a.sel == nullptr) return;
   uint32_t pbeg;
@@ -385,15 +389,15 @@ __device__ __forceinline__ void estimate_item(const EstimateArgs& a, uint32_t b,
   select_item<GROUP>(a, b, h, plan, *tk);
 }
 
-template <int GROUP, bool FUSED>
+template <int GROUP, bool FUSED, uint32_t kPPB = est_kernel_block_pages<GROUP, FUSED>()>
 __global__ __launch_bounds__(kThreads) void estimate_kernel(EstimateArgs a) {
   if constexpr (FUSED) {
     __shared__ EstTopkShared sm;
-    estimate_item<GROUP, true>(a, blockIdx.z, blockIdx.y, blockIdx.x, sm.e, &sm.tk);
+    estimate_item<GROUP, true, kPPB>(a, blockIdx.z, blockIdx.y, blockIdx.x, sm.e, &sm.tk);
   } else {
     __shared__ EstShared sm;
     a.sel = nullptr;
-    estimate_item<GROUP, false>(a, blockIdx.z, blockIdx.y, blockIdx.x, sm, nullptr);
+    estimate_item<GROUP, false, kPPB>(a, blockIdx.z, blockIdx.y, blockIdx.x, sm, nullptr);
   }
 }
 
@@ -1182,12 +1186,17 @@ __global__ void fill_u32_kernel(uint32_t* p, size_t n, uint32_t v) {
 hipError_t launch_estimate(const EstimateArgs& a, uint32_t batch, uint32_t max_pages,
                            hipStream_t s) {
   const bool fused = a.sel != nullptr;
-  const uint32_t ppb = est_kernel_block_pages_of(a.Hq / a.Hkv, fused);
+  uint32_t ppb = est_kernel_block_pages_of(a.Hq / a.Hkv, fused);
+  const bool small =
+      !fused && (uint64_t)((max_pages + ppb - 1u) / ppb) * a.Hkv * batch <= kEstSmallItems;
+  if (small) ppb = kEstSmallPages;
   dim3 grid((max_pages + ppb - 1u) / ppb, a.Hkv, batch);
   switch (a.Hq / a.Hkv) {
 #define AOAKV_EST(G)                                                                   \
   case G:                                                                              \
     if (fused) hipLaunchKernelGGL((estimate_kernel<G, true>), grid, dim3(kThreads), 0, s, a); \
+    else if (small)                                                                           \
+      hipLaunchKernelGGL((estimate_kernel<G, false, kEstSmallPages>), grid, dim3(kThreads), 0, s, a); \
     else hipLaunchKernelGGL((estimate_kernel<G, false>), grid, dim3(kThreads), 0, s, a);      \
     break;
     AOAKV_EST(1)

@@ -892,3 +892,38 @@ def test_one_launch_more_workgroups_than_resident():
     _say("[one launch, 2048 decode items]")
     L = 2007
     _repeated_batch_one_launch(32, L, 1024, [(L - 1) % S + 1] * 8, 93)
+
+
+# items of 16 pages and of 64 (32, 16 with GQA): at and past the count where the
+# scoring launch changes over, rows ending inside an item, each GQA group
+@pytest.mark.parametrize("H,hkv,L", [(32, 32, 8192), (32, 32, 8193), (32, 16, 8000),
+                                     (32, 16, 16500), (16, 4, 1000), (16, 4, 32768 + 17),
+                                     (32, 4, 777), (8, 8, 17)])
+def test_scores_of_every_item_size(H, hkv, L):
+    """decode_estimate against fp64 scores of the stored (fp16) page metadata, and
+    bit for bit against the fused layer's, whose items are of another size."""
+    from aoakv.utils import InferenceController, append_kv, decode_estimate, decode_layer
+    _say(f"[score items] heads={H}/{hkv} L={L}")
+    c = InferenceController(1, H, D, S, 4, L + S, torch.float16, DEV, num_kv_heads=hkv,
+                            shuffle_seed=2)
+    g = torch.Generator(device=DEV).manual_seed(L)
+    k, v = (torch.randn((L, hkv, D), generator=g, device=DEV).half() for _ in range(2))
+    q = torch.randn((1, H, D), generator=g, device=DEV).half()
+    c.prepare_metadata(L)
+    c.begin_forward(L)
+    append_kv(k, v, c, 0)
+    c.begin_forward(1)
+    s = decode_estimate(q, c, 0).clone()
+    P = num_pages(L)
+    pad = lambda x, f: torch.cat([x.double(), x.new_full((P * S - L, hkv, D), f, dtype=torch.float64)]
+                                 ).view(P, S, hkv, D)
+    kmax, kmin = pad(k, -float("inf")).amax(1), pad(k, float("inf")).amin(1)
+    qg = q.double().view(hkv, H // hkv, D)
+    bound = torch.maximum(qg * kmax[:, :, None], qg * kmin[:, :, None]).sum(-1)
+    log_norm = c.v_log_norm_layer(0)[torch.tensor(c.kv_cache.indicies, device=DEV)].double()
+    ref = (torch.logsumexp(2 * bound / math.sqrt(D), -1) + 2 * log_norm).t()
+    assert torch.allclose(s.double(), ref, rtol=2e-6, atol=2e-5)
+    for single in (True, False):
+        c.scores.fill_(float("nan"))
+        decode_layer(q, c, 0, single_launch=single)
+        assert torch.equal(c.scores[0, :, :P], s)
