@@ -138,6 +138,19 @@ constexpr uint32_t kFusedTopkMaxPages = kStageMaxPages;
 // page scores (+ optional fused top-k)
 // ======================================================================
 
+// out[u] = v of lane u of this lane's 16-lane row, u < 8 (DPP row_newbcast)
+__device__ __forceinline__ void row_bcast8(float v, float (&out)[8]) {
+  const int x = __builtin_bit_cast(int, v);
+  out[0] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x150, 0xF, 0xF, false));
+  out[1] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x151, 0xF, 0xF, false));
+  out[2] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x152, 0xF, 0xF, false));
+  out[3] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x153, 0xF, 0xF, false));
+  out[4] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x154, 0xF, 0xF, false));
+  out[5] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x155, 0xF, 0xF, false));
+  out[6] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x156, 0xF, 0xF, false));
+  out[7] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x157, 0xF, 0xF, false));
+}
+
 // Grid (page chunks of 128 / GROUP, kv heads, batch); a wave scores 32 /
 // GROUP consecutive pages, one or (GROUP = 1) two metadata pages (page_size
 // 16), so its metadata page indices are one or two scalar loads.
@@ -259,6 +272,11 @@ __device__ __forceinline__ bool score_item(const EstimateArgs& a, uint32_t b, ui
   const f16 lvn_raw = *(value_aware ? a.v_log_norm + (size_t)phys_j * a.Hkv + hj : a.q);
 
   float sc[kSteps];  // score of step s's page of this row (same in all lanes of the row)
+  // GQA, value-aware: the row's bounds (of step s, query head g: xs[s * GROUP
+  // + g], the same in its 16 lanes)
+  constexpr int kXs = GROUP > 1 ? kSteps * GROUP : 1;
+  static_assert(kXs <= 8, "a lane of a half-row per bound");
+  float xs[kXs];
 #pragma unroll
   for (int s = 0; s < kSteps; ++s) {
     float x[GROUP];
@@ -276,20 +294,12 @@ __device__ __forceinline__ bool score_item(const EstimateArgs& a, uint32_t b, ui
     }
     if (value_aware) {
       // 2 * (bound / sqrt(d)), logsumexp over the group (+ 2 * log-norm below)
-      float m = -INFINITY;
+      if constexpr (GROUP > 1) {
 #pragma unroll
-      for (int g = 0; g < GROUP; ++g) {
-        x[g] = 2.0f * (x[g] / kSqrtHeadDim);
-        m = fmaxf(m, x[g]);
+        for (int g = 0; g < GROUP; ++g) xs[s * GROUP + g] = x[g];
+      } else {
+        sc[s] = 2.0f * (x[0] / kSqrtHeadDim);
       }
-      float lse = x[0];
-      if (GROUP > 1) {
-        float se = 0.f;
-#pragma unroll
-        for (int g = 0; g < GROUP; ++g) se = se + expf(x[g] - m);
-        lse = logf(se) + m;
-      }
-      sc[s] = lse;
     } else {
       float t = x[0];
 #pragma unroll
@@ -298,6 +308,38 @@ __device__ __forceinline__ bool score_item(const EstimateArgs& a, uint32_t b, ui
     }
   }
   const float lvn_lane = (float)lvn_raw;
+  if (GROUP > 1 && value_aware) {
+    // lane l16 % 8 finishes one (step, query head): its division and its
+    // exponential; the logarithm once per step.  With every lane doing the
+    // row's 8 of each (about 250 instructions on an item's chain), estimate,
+    // top-k and attention at 32 / 8 heads, 49000 tokens, took 18.9 us, now 18.1;
+    // 5 sequences' one-launch layer 21.1, now 20.5.  The sum runs over the
+    // heads in order.
+    const uint32_t um = l16 % (uint32_t)kXs, us = um / (uint32_t)GROUP;
+    float x = xs[0];
+#pragma unroll
+    for (int i = 1; i < kXs; ++i) x = um == (uint32_t)i ? xs[i] : x;
+    x = 2.0f * (x / kSqrtHeadDim);
+    float m = fmaxf(x, dpp<kQuadSwap1>(x));
+    if constexpr (GROUP >= 4) m = fmaxf(m, dpp<kQuadSwap2>(m));
+    if constexpr (GROUP == 8) m = fmaxf(m, dpp<kRowHalfMirror>(m));
+    const float e = expf(x - m);
+    float se;
+    if constexpr (GROUP == 2) {
+      se = dpp<0xA0>(e) + dpp<0xF5>(e);  // quad_perm [0,0,2,2], [1,1,3,3]
+    } else if constexpr (GROUP == 4) {
+      se = ((dpp<0x00>(e) + dpp<0x55>(e)) + dpp<0xAA>(e)) + dpp<0xFF>(e);
+    } else {
+      float ev[8];
+      row_bcast8(e, ev);
+      se = ev[0];
+#pragma unroll
+      for (int g = 1; g < 8; ++g) se = se + ev[g];
+    }
+    const float score = (logf(se) + m) + 2.0f * __shfl(lvn_lane, (int)(us * 4u + row));
+    if (l16 < (uint32_t)kXs && um % (uint32_t)GROUP == 0u)
+      s_sc[wave * kPPW + us * kPS + rpage] = score;
+  } else
 #pragma unroll
   for (int s = 0; s < kSteps; ++s) {
     float score = sc[s];
@@ -451,19 +493,6 @@ __global__ __launch_bounds__(kThreads) void topk_kernel(TopkArgs a)
 // ======================================================================
 // sparse decode attention, split-K over pages with a fused merge
 // ======================================================================
-
-// out[u] = v of lane u of this lane's 16-lane row, u < 8 (DPP row_newbcast)
-__device__ __forceinline__ void row_bcast8(float v, float (&out)[8]) {
-  const int x = __builtin_bit_cast(int, v);
-  out[0] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x150, 0xF, 0xF, false));
-  out[1] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x151, 0xF, 0xF, false));
-  out[2] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x152, 0xF, 0xF, false));
-  out[3] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x153, 0xF, 0xF, false));
-  out[4] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x154, 0xF, 0xF, false));
-  out[5] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x155, 0xF, 0xF, false));
-  out[6] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x156, 0xF, 0xF, false));
-  out[7] = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x157, 0xF, 0xF, false));
-}
 
 // out[i] = lane 2i of v's DPP row, in every lane of the row (row_newbcast)
 __device__ __forceinline__ void row_bcast_even8(float v, float (&out)[8]) {
