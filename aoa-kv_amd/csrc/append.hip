@@ -166,7 +166,7 @@ __global__ __launch_bounds__(256) void append_prefill_kernel(AppendPrefillArgs a
   st16(kmax_p, kmax);
   st16(kmin_p, kmin);
   st16(vbar_p, vbar);
-  f16 lvn = log_norm_row(vbar, l16);
+  f16 lvn = log_norm_row(vbar);
   if (l16 == 0u) a.v_log_norm[(size_t)phys * a.H + h] = lvn;
 }
 
@@ -177,6 +177,9 @@ __global__ __launch_bounds__(256) void append_prefill_kernel(AppendPrefillArgs a
 // before the append: RoPE + append + metadata in one launch, the reference's
 // apply_rope_in_place then append_kv_cache_decode (QuestAttention.py:98-111).
 // The new token sits at position L - 1 of its sequence (L counts it).
+// Bound by its chain of round trips and by the rotation's sines: q / k and v are
+// loaded beside the page table and the page's metadata flies during the
+// rotation; with the log-norm's chain in registers, 32 heads 5.7 -> 5.05 us.
 template <bool ROPE>
 __global__ __launch_bounds__(256) void append_decode_kernel(AppendDecodeArgs a) {
   const uint32_t lane = __lane_id();
@@ -191,16 +194,20 @@ __global__ __launch_bounds__(256) void append_decode_kernel(AppendDecodeArgs a) 
   if (h >= (q_block ? a.Hq : a.H)) return;
 
   const uint32_t S = a.S;
+  const uint32_t d0 = l16 * kVec;
+  // q or k, and v, need no earlier load: they go out beside the page table's
+  f16* const x_p = (q_block ? a.q + ((size_t)b * a.Hq + h) * kHeadDim
+                            : a.k + ((size_t)b * a.H + h) * kHeadDim) + d0;
+  const H8 x = ld16(x_p);
+  const H8 vv = ld16(a.v + ((size_t)b * a.H + (q_block ? 0u : h)) * kHeadDim + d0);
   const uint32_t pbeg = (uint32_t)a.kv_indptr[b];
   const uint32_t P = (uint32_t)a.kv_indptr[b + 1] - pbeg;
   const uint32_t lpl = (uint32_t)a.kv_last_page_len[b];
   if (P == 0u || lpl == 0u || lpl > S) return;  // malformed page table: nothing to do
-  RopeTable rt;
+  const uint32_t pos = (P - 1u) * S + lpl - 1u;
   if constexpr (ROPE) {
-    rt = rope_table((P - 1u) * S + lpl - 1u, l16, a.rope_f.f);
     if (q_block) {
-      f16* qp = a.q + ((size_t)b * a.Hq + h) * kHeadDim + l16 * kVec;
-      st16(qp, rope_row(ld16(qp), rt, l16));
+      st16(x_p, rope_row(x, rope_table(pos, l16, a.rope_f.f), l16));
       return;
     }
   }
@@ -209,28 +216,26 @@ __global__ __launch_bounds__(256) void append_decode_kernel(AppendDecodeArgs a) 
   const uint32_t phys = (uint32_t)a.kv_indices[pbeg + p];
   const uint32_t mpage = (uint32_t)a.meta_indices[(uint32_t)a.meta_indptr[b] + p / S];
   const uint32_t ment = p % S;
-  const uint32_t d0 = l16 * kVec;
 
   f16* kmax_p = a.meta + elem_off(a.g, mpage, 0, h, ment) + d0;
   f16* kmin_p = a.meta + elem_off(a.g, mpage, 1, h, ment) + d0;
   f16* vbar_p = a.v_mean + ((size_t)phys * a.H + h) * kHeadDim + d0;
 
-  const size_t in_off = ((size_t)b * a.H + h) * kHeadDim + d0;
-  H8 kk = ld16(a.k + in_off);
-  H8 vv = ld16(a.v + in_off);
-  if constexpr (ROPE) {
-    kk = rope_row(kk, rt, l16);
-    st16(a.k + in_off, kk);
+  H8 kk = x, kmax{}, kmin{}, vbar{};
+  if (e != 0u) {  // (in flight during the rotation)
+    kmax = ld16(kmax_p);
+    kmin = ld16(kmin_p);
+    vbar = ld16(vbar_p);
   }
-  H8 kmax, kmin, vbar;
+  if constexpr (ROPE) {
+    kk = rope_row(x, rope_table(pos, l16, a.rope_f.f), l16);
+    st16(x_p, kk);
+  }
   if (e == 0u) {  // new page: max = min = k, V̄ = v
     kmax = kk;
     kmin = kk;
     vbar = vv;
   } else {
-    kmax = ld16(kmax_p);
-    kmin = ld16(kmin_p);
-    vbar = ld16(vbar_p);
 #pragma unroll
     for (int j = 0; j < kVec; ++j) {
       kmax.v[j] = kk.v[j] > kmax.v[j] ? kk.v[j] : kmax.v[j];
@@ -243,7 +248,7 @@ __global__ __launch_bounds__(256) void append_decode_kernel(AppendDecodeArgs a) 
   st16(kmax_p, kmax);
   st16(kmin_p, kmin);
   st16(vbar_p, vbar);
-  f16 lvn = log_norm_row(vbar, l16);
+  f16 lvn = log_norm_row(vbar);
   if (l16 == 0u) a.v_log_norm[(size_t)phys * a.H + h] = lvn;
 }
 
