@@ -389,9 +389,15 @@ PyObject* prefill_with_paged_kv_cache(PyObject* const* a) {
                  N = (uint32_t)q.size(0), Hq = (uint32_t)q.size(1);
   const Tensor o = a[1] == Py_None ? at::empty_like(q) : THPVariable_Unpack(a[1]);
   // split keys: the chunks' partials, from torch's pool on this stream
-  const size_t n = g_lib.prefill_workspace_size(pages, last, N, causal, Hq, d.D, d.S);
+  size_t n = g_lib.prefill_workspace_size(pages, last, N, causal, Hq, d.D, d.S);
   Tensor ws;
-  if (n != 0) ws = at::empty({(int64_t)n}, q.options().dtype(at::kByte));
+  if (n != 0) {
+    try {
+      ws = at::empty({(int64_t)n}, q.options().dtype(at::kByte));
+    } catch (const c10::OutOfMemoryError&) {
+      n = 0;  // no room (136 MB at most): the call runs unsplit
+    }
+  }
   void* s = stream();
   call("aoakv_prefill_with_paged_kv_cache", [&] {
     return g_lib.prefill_with_workspace(ptr(q), ptr(o), ptr(kv), ix, pages, last, N, causal, Hq,
