@@ -723,8 +723,7 @@ int aoakv_decode_sparse_attn(const void* q, void* o, const void* kv_data,
                           head_dim, page_size, layout, flags))
     return e;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return hip_status(aoakv::tuned_shape(head_dim, page_size) &&
-                            (sel_pages != nullptr || !aoakv::stream_dense(a, batch_size))
+  return hip_status(sel_pages != nullptr && aoakv::tuned_shape(head_dim, page_size)
                         ? aoakv::launch_decode(a, batch_size, s)
                         : aoakv::launch_stream_decode(a, batch_size, head_dim, s),
                     "decode_sparse_attn");

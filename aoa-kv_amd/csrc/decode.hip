@@ -568,8 +568,7 @@ __device__ __forceinline__ void decode_item(const DecodeArgs& a, uint32_t b, uin
   const size_t bh0 = (size_t)b * a.Hq + hq0;  // the item's first query head
   const uint32_t idx0 = chunk * kDecPagesPerBlock + wave * kDecPagesPerWave;
   const uint32_t* sel_row =
-      a.sel ? reinterpret_cast<const uint32_t*>(a.sel) + ((size_t)b * a.Hkv + hkv) * a.sel_stride
-            : nullptr;
+      reinterpret_cast<const uint32_t*>(a.sel) + ((size_t)b * a.Hkv + hkv) * a.sel_stride;
   // Loads are unconditional with clamped addresses and masked afterwards (a
   // load under a lane- or page-dependent condition makes the compiler wait
   // for it before issuing the next).  The page-table words, the selection
@@ -586,14 +585,11 @@ __device__ __forceinline__ void decode_item(const DecodeArgs& a, uint32_t b, uin
   const uint32_t ich = chunk * kDecPagesPerBlock;  // the chunk's first entry
   uint32_t selv[kDecPagesPerWave], sel_ch = 0u;
   if (!HANDOFF) {
-    // dense decode reads its page ids from kv_indices below; its
-    // "selection" loads read kv_indptr[0] (never used)
-    const uint32_t* sel_src = sel_row ? sel_row : reinterpret_cast<const uint32_t*>(a.kv_indptr);
-    const uint32_t sel_last = sel_row ? a.sel_stride - 1u : 0u;
-    sel_ch = ld_agent_u32(sel_src + (ich < sel_last ? ich : sel_last));
+    const uint32_t sel_last = a.sel_stride - 1u;
+    sel_ch = ld_agent_u32(sel_row + (ich < sel_last ? ich : sel_last));
 #pragma unroll
     for (int s = 0; s < kDecPagesPerWave; ++s)
-      selv[s] = ld_agent_u32(sel_src + (idx0 + s < sel_last ? idx0 + s : sel_last));
+      selv[s] = ld_agent_u32(sel_row + (idx0 + s < sel_last ? idx0 + s : sel_last));
   }
   H8 qq[G];
 #pragma unroll
@@ -638,13 +634,10 @@ __device__ __forceinline__ void decode_item(const DecodeArgs& a, uint32_t b, uin
   // physical id of the sequence's last page (the one holding lpl tokens)
   uint32_t last_phys = 0u;
   if constexpr (QUEST) last_phys = (uint32_t)a.kv_indices[pbeg + P - 1u];
-  uint32_t npages = P;
-  if (a.sel != nullptr) {
-    npages = num_selected_pages((P - 1u) * S + lpl, budget, S, P,
-                                QUEST ? kFlagQuestKernel : 0u);
-    const uint32_t row_cap = a.sel_stride + (QUEST ? 1u : 0u);
-    if (npages > row_cap) npages = row_cap;
-  }
+  uint32_t npages = num_selected_pages((P - 1u) * S + lpl, budget, S, P,
+                                       QUEST ? kFlagQuestKernel : 0u);
+  const uint32_t row_cap = a.sel_stride + (QUEST ? 1u : 0u);
+  if (npages > row_cap) npages = row_cap;
   // the grid holds max_chunks blocks per head; never index partials past it
   const uint32_t cap =
       a.max_chunks < (uint32_t)kMergeMaxChunks ? a.max_chunks : (uint32_t)kMergeMaxChunks;
@@ -656,7 +649,7 @@ __device__ __forceinline__ void decode_item(const DecodeArgs& a, uint32_t b, uin
   if (chunk >= nch) return;  // uniform per block
   // entries [0, nsel) come from the selection; with QUEST the entry after
   // them is the last page
-  const uint32_t nsel = (QUEST && a.sel != nullptr) ? npages - 1u : npages;
+  const uint32_t nsel = QUEST ? npages - 1u : npages;
   bool self_topk = false;  // SELF: the entries came from this workgroup's top-k
   if constexpr (SELF) {
     // the head's selection, computed here: entries [0, nout), in page order
@@ -710,13 +703,8 @@ __device__ __forceinline__ void decode_item(const DecodeArgs& a, uint32_t b, uin
 #pragma unroll
   for (int s = 0; s < kDecPagesPerWave; ++s) {
     live[s] = idx0 + s < npages;
-    if (a.sel != nullptr) {
-      phys[s] = live[s] ? selv[s] : sel_ch;
-      if (QUEST && idx0 + s >= nsel) phys[s] = last_phys;
-    } else {
-      const uint32_t i = live[s] ? idx0 + s : ich;
-      phys[s] = (uint32_t)a.kv_indices[pbeg + i];
-    }
+    phys[s] = live[s] ? selv[s] : sel_ch;
+    if (QUEST && idx0 + s >= nsel) phys[s] = last_phys;
   }
   // STREAM (no GQA: each selected page's K/V is read by this item alone):
   // non-temporal loads, config 2 21.33 -> 20.88 us per layer.  The query

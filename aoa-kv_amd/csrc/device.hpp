@@ -15,6 +15,7 @@ namespace aoakv {
 using f16 = _Float16;
 
 constexpr int kWave = 64;
+constexpr uint32_t kXcds = 8;  // MI355X: 8 XCDs, workgroups dealt to them round-robin
 constexpr int kHeadDim = 128;
 constexpr int kPageSize = 16;
 constexpr int kLanesPerRow = 16;   // lanes covering one 128-dim fp16 vector

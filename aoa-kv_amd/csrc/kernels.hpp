@@ -159,7 +159,7 @@ struct DecodeArgs {
   const int32_t* kv_indptr;
   const int32_t* kv_indices;
   const int32_t* kv_last_page_len;
-  const int32_t* sel;  // [B, Hkv, sel_stride] physical ids, or nullptr (dense)
+  const int32_t* sel;  // [B, Hkv, sel_stride] physical ids, or nullptr (dense: stream.hip only)
   uint32_t sel_stride;
   uint32_t token_budget;
   const int32_t* token_budgets;
@@ -258,7 +258,6 @@ uint32_t layer_self_blocks_per_cu(uint32_t group, uint32_t heads_per_item, uint3
 
 // stream.hip: dense decode (a.sel == nullptr, any shape), and the selected
 // pages of the shapes without tuned kernels
-bool stream_dense(const DecodeArgs& a, uint32_t batch);  // the tuned shape's, else decode.hip
 // self: the decode selects for itself, as launch_decode's (where stream_selects
 // says so)
 bool stream_selects(const DecodeArgs& a, uint32_t batch, uint32_t max_pages);

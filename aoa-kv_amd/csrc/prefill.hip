@@ -47,7 +47,6 @@ constexpr int kPfQueriesPerWave = 32;
 constexpr int kPfQueriesPerBlock = 128;
 constexpr int kPfTileKeys = 64;
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr uint32_t kXcds = 8;  // MI355X: 8 XCDs, workgroups dealt to them round-robin
 
 __device__ inline floatx16 mfma32(const half8& a, const half8& b, const floatx16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);

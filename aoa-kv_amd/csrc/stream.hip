@@ -14,11 +14,12 @@
 // of its own tokens: nothing crosses groups until the end.
 //
 // Bound by HBM for long lists, else by the chain of a workgroup's round trips
-// (page table, ids, K/V, partials, merge).  Two layers, before (a workgroup
-// per 8 pages) and now: 16384 tokens x 32 heads 121 -> 98 us (5.5 TB/s; a
-// plain read of 1 GiB runs at 6.05), 32 / 8 heads at 24000 118 -> 62, head
-// dim 64 at 20000 153 -> 63, 256 (16 heads) at 8000 95 -> 58; one selected
-// layer of 128 pages x 16 heads of dim 256 (decode alone) 16.2 -> 13.3.
+// (page table, ids, K/V, partials, merge).  Two layers, with a workgroup per 8
+// pages and now: 16384 tokens x 32 heads 121 -> 91 us (5.9 TB/s; a plain read
+// of 1 GiB runs at 6.05), 1000 tokens 14.7 -> 14.3, 32 / 8 heads at 24000 117
+// -> 60, head dim 64 at 20000 151 -> 61, 256 (16 heads) at 8000 92 -> 54; one
+// selected layer of 128 pages x 16 heads of dim 256 (decode alone) 16.2 ->
+// 13.3.
 #include "kernels.hpp"
 #include "topk.hpp"
 
@@ -89,34 +90,127 @@ __device__ inline float logit_f16(float x) {
   return (float)r16(x * (D == 64 ? 0.125f : 0.0625f));
 }
 
-// A call, and its split: chunks the grid holds per head (<= max_chunks), and
-// the factor that divides by the page size (0: pages of one token).
+// Which pages a kernel attends: all (dense), the call's selection rows, or (for
+// a layer) the selection it makes itself from the scores.
+enum Pages { kAll, kListed, kSelf };
+
+// A call and its split.
 struct StreamArgs : DecodeArgs {
-  uint32_t grid_chunks;
-  uint32_t page_rcp;
-  // SELF: the rows the selection is made from (complete), and where it goes
+  uint32_t page_rcp;  // the factor that divides by the page size (0: pages of one token)
+  // kAll: the chunks the call's pages are cut into (per head, over all its
+  // sequences), below and from long_pages pages of all sequences on, and the
+  // factors that divide by these numbers (0: by one)
+  uint32_t batch;
+  uint32_t split, split_rcp, long_split, long_rcp;
+  uint32_t long_pages;
+  // kSelf: the rows the selection is made from (complete), and where it goes
   const float* scores;
   uint32_t score_stride;
   uint32_t select_flags;
   int32_t* sel_out;
 };
 
-// One workgroup per (chunk of the page list, G query heads of a kv head,
-// sequence).  G: 1, or the whole GQA group, whose K/V is then loaded once.
-// The list is split over a.grid_chunks chunks (of at least kGenChunkPages
-// pages); the last to arrive at the head's counter merges their partials in
-// chunk order and clears them.
+// ceil(n / d) for 1 <= n, rcp = floor(2^32 / d) + 1 (0: d = 1); from n * d = 2^32
+// on it may be more
+__device__ inline uint32_t div_up(uint32_t n, uint32_t rcp) {
+  return rcp == 0u ? n : (uint32_t)(((uint64_t)(n - 1u) * rcp) >> 32) + 1u;
+}
+
+// Where a workgroup of a dense call works: sequence b's chunk `chunk` of `per`
+// pages, with b's place in the page table.
+struct Place {
+  uint32_t b, chunk, per, pbeg, pages, last_len;
+};
+
+// Pages per chunk of a call of `total` pages.  (The bound matters only for more
+// than 64 sequences with page tables past it, which `total` counts whole.)
+__device__ inline uint32_t chunk_pages(const StreamArgs& a, uint32_t total) {
+  const bool is_long =
+      total >= a.long_pages && (uint64_t)a.max_pages * a.batch >= a.long_pages;
+  const uint32_t per = is_long ? div_up(total, a.long_rcp) : div_up(total, a.split_rcp);
+  return per < kGenChunkPages ? kGenChunkPages : per;
+}
+
+// The item-th chunk of the call: sequences in order, each one's chunks in order.
+// No pages: there is none.
+__device__ inline Place find_item(const StreamArgs& a, uint32_t item) {
+  const uint32_t lane = __lane_id();
+  if (a.batch == 1u) {
+    const uint32_t beg = (uint32_t)a.kv_indptr[0], n = (uint32_t)a.kv_indptr[1] - beg;
+    const uint32_t len = (uint32_t)a.kv_last_page_len[0];
+    const uint32_t P = n < a.max_pages ? n : a.max_pages;
+    return Place{0u, item, chunk_pages(a, P != 0u ? P : 1u), beg, n, len};
+  }
+  auto of = [](uint32_t x, uint32_t j) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, (int)j);
+  };
+  if (a.batch <= (uint32_t)kWave) {  // a lane per sequence, their chunks counted
+    const uint32_t i = lane < a.batch ? lane : a.batch - 1u;
+    const uint32_t beg = (uint32_t)a.kv_indptr[i], end = (uint32_t)a.kv_indptr[i + 1u];
+    const uint32_t len = (uint32_t)a.kv_last_page_len[i];
+    uint32_t P = end - beg < a.max_pages ? end - beg : a.max_pages;
+    if (lane >= a.batch) P = 0u;
+    const uint32_t total = of(wave_incl_scan(P), kWave - 1u);
+    if (total == 0u) return Place{};
+    const uint32_t per = chunk_pages(a, total);
+    const uint32_t n = (P + per - 1u) / per;
+    const uint32_t incl = wave_incl_scan(n);
+    const uint64_t past = __builtin_amdgcn_ballot_w64(item < incl);
+    if (past == 0u) return Place{};
+    const uint32_t j = (uint32_t)__builtin_ctzll(past);
+    return Place{j, item - (of(incl, j) - of(n, j)), per, of(beg, j), of(end, j) - of(beg, j),
+                 of(len, j)};
+  }
+  // more: sequence b's items start at floor(pages before it / per) + b, room
+  // for its chunks whatever the lengths, so only its own place is needed; 64
+  // sequences are tried at a time
+  const uint32_t first = (uint32_t)a.kv_indptr[0];
+  const uint32_t total = (uint32_t)a.kv_indptr[a.batch] - first;
+  if (total == 0u) return Place{};
+  const uint32_t per = chunk_pages(a, total);
+  uint32_t lo = 0u, n = a.batch;
+  for (;;) {
+    const uint32_t stride = (n + kWave - 1u) / kWave;
+    const bool in = lane * stride < n;
+    const uint32_t i = in ? lo + lane * stride : lo;
+    const uint32_t beg = (uint32_t)a.kv_indptr[i], end = (uint32_t)a.kv_indptr[i + 1u];
+    const uint32_t len = (uint32_t)a.kv_last_page_len[i];
+    const uint32_t off = (beg - first) / per + i;
+    const uint64_t le = __builtin_amdgcn_ballot_w64(in && off <= item);
+    if (le == 0u) return Place{};  // malformed page table
+    const uint32_t j = 63u - (uint32_t)__builtin_clzll(le);
+    if (stride == 1u)
+      return Place{lo + j, item - of(off, j), per, of(beg, j), of(end, j) - of(beg, j),
+                   of(len, j)};
+    const uint32_t left = n - j * stride;
+    n = left < stride ? left : stride;
+    lo += j * stride;
+  }
+}
+
+// One workgroup per (chunk of the page list, G query heads of a kv head).  G:
+// 1, or the whole GQA group, whose K/V is then loaded once.
+// kAll: the pages of all sequences are cut into as many chunks per head as
+// fill the chip (each sequence into chunks of that many pages, at least
+// kGenChunkPages), a count made here from the page table: what a call gives
+// depends on its sequences alone, not on the page count it was sized for, nor on
+// G.  Selected pages are cut into chunks of kGenChunkPages.  The last chunk of a
+// sequence to arrive at the head's counter merges the partials in chunk
+// order and clears them.
 // NT: no other workgroup reads these pages: non-temporal loads.
-// SELF: there are no selection rows yet; every workgroup of a kv head runs the
+// kSelf: there are no selection rows yet; every workgroup of a kv head runs the
 // head's top-k on the scores the previous launch wrote, takes its chunk's
 // entries and writes them out (as decode.hip's two-launch layer).
-template <int D, int G, bool NT, bool SELF = false>
+template <int D, int G, bool NT, Pages PAGES>
 __global__ __launch_bounds__(kStThreads) void stream_decode_kernel(StreamArgs a) {
+  constexpr bool SELF = PAGES == kSelf;
   constexpr uint32_t N = D / 8, GPW = kWave / N;  // lanes per group, groups per wave
   constexpr uint32_t kBatch = kU * GPW;           // tokens
-  // two batches in flight: 128 registers, four waves per SIMD; three (168)
-  // were slower at every shape measured (16 sequences' d64 layer 43.0
-  // against 38.5 us, pages of 8 127.8 against 115.1 per 4 layers)
+  // two batches in flight; three were slower at every shape measured (16
+  // sequences' d64 layer 43.0 against 38.5 us, pages of 8 127.8 against
+  // 115.1 per 4 layers).  Registers, and waves per SIMD: selected pages 128
+  // and 4, every page 140 and 3; groups of 2, 4 and 8 heads 146, 188 and 256
+  // (with 16 spilled to AGPRs), and 3, 2 and 1
   constexpr int kAhead = 2;
   constexpr uint32_t kStride = (uint32_t)D + 4u;  // partial: o[D], m, l, pad
   struct Shared {
@@ -135,22 +229,45 @@ __global__ __launch_bounds__(kStThreads) void stream_decode_kernel(StreamArgs a)
   const uint32_t lane = __lane_id();
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint32_t l = lane % N, v = lane / N;
-  // dense: heads fastest, so the workgroups in flight read whole pages
-  // (neighbouring heads are neighbours in HBM); else chunks fastest
-  const uint32_t chunk = a.sel == nullptr ? blockIdx.y : blockIdx.x;
-  const uint32_t hq0 = (a.sel == nullptr ? blockIdx.x : blockIdx.y) * G, b = blockIdx.z;
-  const uint32_t hkv = hq0 / (a.Hq / a.Hkv);
-  const bool quest = (a.flags & kFlagQuestKernel) != 0u;
+  const bool quest = PAGES != kAll && (a.flags & kFlagQuestKernel) != 0u;
   const uint32_t S = a.S;
-  const uint32_t pbeg = (uint32_t)a.kv_indptr[b];
-  const uint32_t P_table = (uint32_t)a.kv_indptr[b + 1] - pbeg;
-  const uint32_t P = P_table < a.max_pages ? P_table : a.max_pages;
-  if (P != P_table && chunk == 0u && threadIdx.x == 0u) flag_error(a.error, kErrTruncated);
-  const uint32_t lpl = (uint32_t)a.kv_last_page_len[b];
+  uint32_t chunk, hq0, hkv, per = kGenChunkPages;
+  Place at;
+  if constexpr (PAGES == kAll) {
+    // heads fastest, so the workgroups in flight read whole pages
+    // (neighbouring heads are neighbours in HBM)
+    uint32_t item = blockIdx.y + gridDim.y * blockIdx.z;
+    if constexpr (G > 1 || NT) {
+      hkv = blockIdx.x;
+      hq0 = hkv * G;
+    } else {
+      // the heads of a GQA group on one XCD (workgroup x runs on x % 8), which
+      // reads their K/V from HBM once: 32 / 8 heads, two layers at 2000 tokens
+      // 23.7 -> 15.2 us
+      const uint32_t group = a.Hq / a.Hkv, x = blockIdx.x + a.Hq * item;
+      const uint32_t u = x / (kXcds * group) * kXcds + x % kXcds;
+      hkv = u % a.Hkv;
+      hq0 = hkv * group + x / kXcds % group;
+      item = u / a.Hkv;
+    }
+    at = find_item(a, item);
+    per = at.per;
+    chunk = at.chunk;
+  } else {
+    chunk = blockIdx.x;
+    hq0 = blockIdx.y * G;
+    hkv = hq0 / (a.Hq / a.Hkv);
+    const uint32_t b = blockIdx.z, beg = (uint32_t)a.kv_indptr[b];
+    at = Place{b, chunk, per, beg, (uint32_t)a.kv_indptr[b + 1u] - beg,
+               (uint32_t)a.kv_last_page_len[b]};
+  }
+  const uint32_t b = at.b, pbeg = at.pbeg, lpl = at.last_len;
+  const uint32_t P = at.pages < a.max_pages ? at.pages : a.max_pages;
+  if (P != at.pages && chunk == 0u && threadIdx.x == 0u) flag_error(a.error, kErrTruncated);
   if (P == 0u || lpl == 0u || lpl > S) return;  // malformed page table
-  const uint32_t budget = a.token_budgets ? (uint32_t)a.token_budgets[b] : a.token_budget;
-  uint32_t npages = P;
-  if (a.sel != nullptr) {
+  uint32_t npages = P, budget = 0u;
+  if constexpr (PAGES != kAll) {
+    budget = a.token_budgets ? (uint32_t)a.token_budgets[b] : a.token_budget;
     npages = num_selected_pages((P - 1u) * S + lpl, budget, S, P, quest ? kFlagQuestKernel : 0u);
     const uint32_t row_cap = a.sel_stride + (quest ? 1u : 0u);
     if (npages > row_cap) npages = row_cap;
@@ -160,12 +277,10 @@ __global__ __launch_bounds__(kStThreads) void stream_decode_kernel(StreamArgs a)
     npages = a.max_chunks * kGenChunkPages;
     if (chunk == 0u && threadIdx.x == 0u) flag_error(a.error, kErrTruncated);
   }
-  uint32_t per = (npages + a.grid_chunks - 1u) / a.grid_chunks;  // pages per chunk
-  if (per < kGenChunkPages) per = kGenChunkPages;
-  const uint32_t nch = (npages + per - 1u) / per;
-  if (chunk >= nch) return;  // uniform per block
-  const uint32_t nsel = (quest && a.sel != nullptr) ? npages - 1u : npages;
-  const int32_t* sel_row = a.sel ? a.sel + ((size_t)b * a.Hkv + hkv) * a.sel_stride : nullptr;
+  if (chunk * per >= npages) return;  // uniform per block
+  const uint32_t nsel = quest ? npages - 1u : npages;
+  const int32_t* sel_row =
+      PAGES == kListed ? a.sel + ((size_t)b * a.Hkv + hkv) * a.sel_stride : nullptr;
   const uint32_t last_phys = (uint32_t)a.kv_indices[pbeg + P - 1u];
   const size_t bh0 = (size_t)b * a.Hq + hq0;
   H8 q[G];
@@ -207,7 +322,7 @@ __global__ __launch_bounds__(kStThreads) void stream_decode_kernel(StreamArgs a)
       if (i < nsel && i >= nout) flag_error(a.error, kErrTruncated);
       s_page[threadIdx.x] = i >= nsel ? last_phys : i < nout ? entry(i) : last_phys;
     }
-    const uint32_t o_end = chunk == nch - 1u || i0 + per > nout ? nout : i0 + per;
+    const uint32_t o_end = i1 == npages || i0 + per > nout ? nout : i0 + per;
     for (uint32_t i = i0 + threadIdx.x; i < o_end; i += kStThreads) out[i] = (int32_t)entry(i);
     __syncthreads();  // (the top-k's memory is the softmax's from here)
   }
@@ -217,9 +332,9 @@ __global__ __launch_bounds__(kStThreads) void stream_decode_kernel(StreamArgs a)
     if constexpr (!SELF) {
       if (ib != i0) __syncthreads();  // the ids before were read
       for (uint32_t i = threadIdx.x; i < np; i += kStThreads)
-        s_page[i] = sel_row == nullptr ? (uint32_t)a.kv_indices[pbeg + ib + i]
-                    : ib + i < nsel    ? (uint32_t)sel_row[ib + i]
-                                       : last_phys;
+        s_page[i] = PAGES == kAll    ? (uint32_t)a.kv_indices[pbeg + ib + i]
+                    : ib + i < nsel ? (uint32_t)sel_row[ib + i]
+                                    : last_phys;
       __syncthreads();
     }
     const uint32_t T = np * S;  // token slots
@@ -244,59 +359,85 @@ __global__ __launch_bounds__(kStThreads) void stream_decode_kernel(StreamArgs a)
         if (t < T && (phys != last_phys || slot < lpl)) ok[s] |= 1u << u;
       }
     };
+    auto attend = [&](int s) {
+      // slots without a token hold whatever the cache held: 0 * NaN is NaN
+      if (__builtin_amdgcn_ballot_w64(ok[s] != (1u << kU) - 1u) != 0u) {
 #pragma unroll
-    for (int s = 0; s < kAhead; ++s) load(wave + (uint32_t)s * kStWaves, s);
-    for (uint32_t i = wave; i < nb; i += kAhead * kStWaves) {
+        for (int u = 0; u < kU; ++u)
+          if (!((ok[s] >> u) & 1u)) vv[s][u] = H8{};
+      }
 #pragma unroll
-      for (int s = 0; s < kAhead; ++s) {
-        if (i + (uint32_t)s * kStWaves >= nb) break;  // wave-uniform
-        // slots without a token hold whatever the cache held: 0 * NaN is NaN
-        if (__builtin_amdgcn_ballot_w64(ok[s] != (1u << kU) - 1u) != 0u) {
+      for (int g = 0; g < G; ++g) {
+        float x[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+          float acc = 0.f;
+#pragma unroll
+          for (int p = 0; p < kVec / 2; ++p)
+            acc = __builtin_amdgcn_fdot2(half_pair(q[g], p), half_pair(kk[s][u], p), acc, false);
+          x[u] = lanes_sum<D>(acc);
+        }
+        // lane l % 4 rounds and exponentiates token l % 4
+        const uint32_t um = lane % 4u;
+        float pick = x[0];
+#pragma unroll
+        for (int u = 1; u < kU; ++u) pick = um == (uint32_t)u ? x[u] : pick;
+        float xm = logit_f16<D>((float)r16(pick));
+        xm = (ok[s] >> um) & 1u ? xm : -INFINITY;
+        float mt = fmaxf(xm, dpp<kQuadSwap1>(xm));
+        mt = fmaxf(mt, dpp<kQuadSwap2>(mt));
+        const float mn = fmaxf(m[g], mt);
+        const float c = __expf(m[g] - mn), p = __expf(xm - mn);
+        m[g] = mn;
+        float ps = p + dpp<kQuadSwap1>(p);
+        ps = ps + dpp<kQuadSwap2>(ps);
+        lsum[g] = lsum[g] * c + ps;
+        const float pv[kU] = {quad_bcast<0>(p), quad_bcast<1>(p), quad_bcast<2>(p),
+                              quad_bcast<3>(p)};
+#pragma unroll
+        for (int j = 0; j < kVec; ++j) {
+          float acc = o[g][j] * c;
 #pragma unroll
           for (int u = 0; u < kU; ++u)
-            if (!((ok[s] >> u) & 1u)) vv[s][u] = H8{};
+            acc = __builtin_fmaf(pv[u], (float)vv[s][u].v[j], acc);
+          o[g][j] = acc;
         }
+      }
+    };
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-          float x[kU];
-#pragma unroll
-          for (int u = 0; u < kU; ++u) {
-            float acc = 0.f;
-#pragma unroll
-            for (int p = 0; p < kVec / 2; ++p)
-              acc = __builtin_amdgcn_fdot2(half_pair(q[g], p), half_pair(kk[s][u], p), acc, false);
-            x[u] = lanes_sum<D>(acc);
-          }
-          // lane l % 4 rounds and exponentiates token l % 4
-          const uint32_t um = lane % 4u;
-          float pick = x[0];
-#pragma unroll
-          for (int u = 1; u < kU; ++u) pick = um == (uint32_t)u ? x[u] : pick;
-          float xm = logit_f16<D>((float)r16(pick));
-          xm = (ok[s] >> um) & 1u ? xm : -INFINITY;
-          float mt = fmaxf(xm, dpp<kQuadSwap1>(xm));
-          mt = fmaxf(mt, dpp<kQuadSwap2>(mt));
-          const float mn = fmaxf(m[g], mt);
-          const float c = __expf(m[g] - mn), p = __expf(xm - mn);
-          m[g] = mn;
-          float ps = p + dpp<kQuadSwap1>(p);
-          ps = ps + dpp<kQuadSwap2>(ps);
-          lsum[g] = lsum[g] * c + ps;
-          const float pv[kU] = {quad_bcast<0>(p), quad_bcast<1>(p), quad_bcast<2>(p),
-                                quad_bcast<3>(p)};
-#pragma unroll
-          for (int j = 0; j < kVec; ++j) {
-            float acc = o[g][j] * c;
-#pragma unroll
-            for (int u = 0; u < kU; ++u)
-              acc = __builtin_fmaf(pv[u], (float)vv[s][u].v[j], acc);
-            o[g][j] = acc;
-          }
+    for (int s = 0; s < kAhead; ++s) load(wave + (uint32_t)s * kStWaves, s);
+    uint32_t i = wave;
+    if constexpr (PAGES == kAll && G == 1) {
+      // no load past the list's end, for which a short list would wait at its
+      // own (two layers of 32 heads, 500 tokens 13.3 -> 11.2 us); three waves per
+      // SIMD instead of four, no slower on long lists
+      static_assert(kAhead == 2, "the loop's exits");
+      for (; i < nb; i += 2u * kStWaves) {
+        attend(0);
+        if (i + 2u * kStWaves >= nb) {
+          if (i + kStWaves < nb) attend(1);
+          break;
         }
-        load(i + (uint32_t)(s + kAhead) * kStWaves, s);
+        load(i + 2u * kStWaves, 0);
+        attend(1);
+        if (i + 3u * kStWaves >= nb) {
+          attend(0);
+          break;
+        }
+        load(i + 3u * kStWaves, 1);
+      }
+    } else {
+      for (; i < nb; i += kAhead * kStWaves) {
+#pragma unroll
+        for (int s = 0; s < kAhead; ++s) {
+          if (i + (uint32_t)s * kStWaves >= nb) break;  // wave-uniform
+          attend(s);
+          load(i + (uint32_t)(s + kAhead) * kStWaves, s);
+        }
       }
     }
   }
+  const uint32_t nch = (npages + per - 1u) / per;
 
   // ---- the wave's groups, then the workgroup's waves
 #pragma unroll
@@ -342,37 +483,42 @@ __global__ __launch_bounds__(kStThreads) void stream_decode_kernel(StreamArgs a)
   }
   if (nch == 1u) return;
   if (!arrive_last(&a.counters[bh0 * kCounterStride], nch, &s_last)) return;
-  // the last chunk to arrive merges: in groups of 16 chunks, every load of a
+  // the last chunk to arrive merges: in groups of kC chunks, every load of a
   // group issued before any is used, folded in chunk order
-  for (uint32_t x = threadIdx.x; x < (uint32_t)(G * D); x += kStThreads) {
-    const uint32_t g = x / D, d = x % D;
-    const float* base = a.partial + (bh0 + g) * a.max_chunks * kStride;
-    float M = kNoMax, Ls = 0.f, acc = 0.f;
-    for (uint32_t c0 = 0; c0 < nch; c0 += 16u) {
-      float mc[16], lc[16], oc[16];
+  auto merge = [&](auto group) {
+    constexpr uint32_t kC = decltype(group)::value;
+    for (uint32_t x = threadIdx.x; x < (uint32_t)(G * D); x += kStThreads) {
+      const uint32_t g = x / D, d = x % D;
+      const float* base = a.partial + (bh0 + g) * a.max_chunks * kStride;
+      float M = kNoMax, Ls = 0.f, acc = 0.f;
+      for (uint32_t c0 = 0; c0 < nch; c0 += kC) {
+        float mc[kC], lc[kC], oc[kC];
 #pragma unroll
-      for (uint32_t u = 0; u < 16u; ++u) {
-        const float* part = base + (c0 + u < nch ? c0 + u : nch - 1u) * kStride;
-        mc[u] = ld_agent(part + D);
-        lc[u] = ld_agent(part + D + 1u);
-        oc[u] = ld_agent(part + d);
+        for (uint32_t u = 0; u < kC; ++u) {
+          const float* part = base + (c0 + u < nch ? c0 + u : nch - 1u) * kStride;
+          mc[u] = ld_agent(part + D);
+          lc[u] = ld_agent(part + D + 1u);
+          oc[u] = ld_agent(part + d);
+        }
+        float Mn = M;
+#pragma unroll
+        for (uint32_t u = 0; u < kC; ++u) Mn = fmaxf(Mn, mc[u]);
+        const float keep = __expf(M - Mn);
+        Ls = Ls * keep;
+        acc = acc * keep;
+#pragma unroll
+        for (uint32_t u = 0; u < kC; ++u) {
+          const float w = c0 + u < nch ? __expf(mc[u] - Mn) : 0.f;
+          Ls = Ls + w * lc[u];
+          acc = acc + w * oc[u];
+        }
+        M = Mn;
       }
-      float Mn = M;
-#pragma unroll
-      for (uint32_t u = 0; u < 16u; ++u) Mn = fmaxf(Mn, mc[u]);
-      const float keep = __expf(M - Mn);
-      Ls = Ls * keep;
-      acc = acc * keep;
-#pragma unroll
-      for (uint32_t u = 0; u < 16u; ++u) {
-        const float w = c0 + u < nch ? __expf(mc[u] - Mn) : 0.f;
-        Ls = Ls + w * lc[u];
-        acc = acc + w * oc[u];
-      }
-      M = Mn;
+      a.o[(bh0 + g) * D + d] = r16(acc / Ls);
     }
-    a.o[(bh0 + g) * D + d] = r16(acc / Ls);
-  }
+  };
+  if (nch <= 8u) merge(std::integral_constant<uint32_t, 8u>{});
+  else merge(std::integral_constant<uint32_t, 16u>{});
   __syncthreads();  // every thread has read the partials
   for (uint32_t g = 0; g < (uint32_t)G; ++g) {
     uint32_t* pw = reinterpret_cast<uint32_t*>(a.partial + (bh0 + g) * a.max_chunks * kStride);
@@ -383,46 +529,56 @@ __global__ __launch_bounds__(kStThreads) void stream_decode_kernel(StreamArgs a)
 template <int D>
 hipError_t launch_d(const StreamArgs& a, uint32_t G, dim3 grid, hipStream_t s) {
   const dim3 block(kStThreads);
+  const bool mha = a.Hq == a.Hkv;
+#define AOAKV_ST(G_, NT_, PAGES_) \
+  hipLaunchKernelGGL((stream_decode_kernel<D, G_, NT_, PAGES_>), grid, block, 0, s, a)
   if (a.scores != nullptr) {
-    if (a.Hq == a.Hkv)
-      hipLaunchKernelGGL((stream_decode_kernel<D, 1, true, true>), grid, block, 0, s, a);
-    else
-      hipLaunchKernelGGL((stream_decode_kernel<D, 1, false, true>), grid, block, 0, s, a);
-    return hipGetLastError();
-  }
-  // K/V of one reader: no GQA group, or a whole group per workgroup
-  if (G > 1u || a.Hq == a.Hkv) {
+    if (mha) AOAKV_ST(1, true, kSelf);
+    else AOAKV_ST(1, false, kSelf);
+  } else if (a.sel != nullptr) {
+    if (mha) AOAKV_ST(1, true, kListed);
+    else AOAKV_ST(1, false, kListed);
+  } else {
+    // K/V of one reader: no GQA group, or a whole group per workgroup
     switch (G) {
-      case 1: hipLaunchKernelGGL((stream_decode_kernel<D, 1, true>), grid, block, 0, s, a); break;
-      case 2: hipLaunchKernelGGL((stream_decode_kernel<D, 2, true>), grid, block, 0, s, a); break;
-      case 4: hipLaunchKernelGGL((stream_decode_kernel<D, 4, true>), grid, block, 0, s, a); break;
-      case 8: hipLaunchKernelGGL((stream_decode_kernel<D, 8, true>), grid, block, 0, s, a); break;
+      case 1:
+        if (mha) AOAKV_ST(1, true, kAll);
+        else AOAKV_ST(1, false, kAll);
+        break;
+      case 2: AOAKV_ST(2, true, kAll); break;
+      case 4: AOAKV_ST(4, true, kAll); break;
+      case 8: AOAKV_ST(8, true, kAll); break;
       default: return hipErrorInvalidValue;
     }
-  } else {
-    hipLaunchKernelGGL((stream_decode_kernel<D, 1, false>), grid, block, 0, s, a);
   }
+#undef AOAKV_ST
   return hipGetLastError();
 }
 
 }  // namespace
 
-// Query heads per workgroup of a dense call: the whole GQA group, whose K/V is
-// then read once, when that still gives the chip 512 workgroups of 8 pages;
-// below, a head each (their partials are merged in parallel).  32 / 8 heads,
-// two layers: 12000 tokens 82 us a head each (decode.hip's kernel), 45
-// grouped; 5000 tokens 27 and 35.
-static uint32_t dense_group(const DecodeArgs& a, uint32_t batch) {
-  return (uint64_t)a.max_chunks * a.Hkv * batch >= 512u ? a.Hq / a.Hkv : 1u;
-}
-
-// The dense calls of the tuned shape that stream: without GQA from 1024
-// workgroups of 8 pages on.  Two layers of 32 heads: 3000 tokens (752) 28.0
-// us streamed, 27.9 by decode.hip's kernel, 5000 (1280) 38.6 and 44.6, 16384
-// 98 and 122 (5.5 and 4.4 TB/s), 24000 137 and 181.
-bool stream_dense(const DecodeArgs& a, uint32_t batch) {
-  return dense_group(a, batch) > 1u ||
-         (a.Hq == a.Hkv && (uint64_t)a.max_chunks * a.Hq * batch >= 1024u);
+// Dense calls are cut into 512 workgroups (2 per CU, and no fewer than 8 pages
+// each), which stream 32 heads of 16384 tokens at 5.9 TB/s; more of them cost
+// more partials (1024: 25.5 -> 32 us at 3000 tokens, 92 -> 96 at 16384).  The
+// heads of a GQA group read their K/V through one XCD's L2, at 12 to 17 TB/s
+// whatever the group.  A workgroup for the whole group reads it at HBM's 6
+// TB/s, but takes its heads one after the other (one workgroup per CU, 256 in
+// all), 11 to 34 us before that shows.  So a call is long, and read by
+// groups, from 256 MiB of L2 reads on (more where fewer than 8 kv heads make
+// more and shorter chunks).  Two layers, a head and a group per workgroup:
+// 32 / 8 heads at 5000 tokens 21 and 33 us, 12000 36 and 43, 24000 60 and 59,
+// 65536 153 and 114; 32 / 16 at 10000 37 and 40, 20000 72 and 66; 32 / 4 at
+// 40000 88 and 106, 65536 133 and 130; head dim 64, 32 / 8 at 30000 42 and 42;
+// 256, 16 / 8 at 20000 74 and 74.
+// The chunks come from the tokens there are.  Made from the call's bound and
+// its batch, one sequence of 65536 tokens among 15 of 1000 (32 heads) took 1770
+// us, now 423, and among 31 (32 / 8 heads) 2545, now 161.
+// Pages of all sequences from which a call is long:
+static uint32_t dense_long_pages(const DecodeArgs& a, uint32_t head_dim) {
+  if (a.Hq == a.Hkv) return ~0u;
+  const uint64_t bytes = (uint64_t)(256u << 20) * (a.Hkv < 8u ? 8u / a.Hkv : 1u);
+  const uint64_t page = 4ull * head_dim * a.Hq * a.S;
+  return (uint32_t)((bytes + page - 1u) / page);
 }
 
 // The layers whose decode selects for itself: rows the top-k stages, and no
@@ -445,18 +601,30 @@ hipError_t launch_stream_decode(const DecodeArgs& args, uint32_t batch, uint32_t
     a.select_flags = self->flags;
     a.sel_out = self->sel;
   }
-  a.page_rcp = a.S > 1u ? (uint32_t)((1ull << 32) / a.S) + 1u : 0u;
-  const bool dense = a.sel == nullptr;
-  const uint32_t G = dense ? dense_group(a, batch) : 1u, heads = a.Hq / G;
-  a.grid_chunks = a.max_chunks;
-  if (dense) {
-    // a workgroup per CU (two without GQA), each a long stream: the partials
-    // and their merge shrink with the chunks (32 / 8 heads, 24000 tokens: 89
-    // us with 768 workgroups, 72 with 512, 62 with 256)
-    const uint64_t want = (G > 1u ? 256u : 512u) / ((uint64_t)heads * batch);
-    a.grid_chunks = want < 1u ? 1u : want < a.max_chunks ? (uint32_t)want : a.max_chunks;
+  auto rcp = [](uint32_t d) { return d > 1u ? (uint32_t)((1ull << 32) / d) + 1u : 0u; };
+  a.page_rcp = rcp(a.S);
+  uint32_t G = 1u;
+  dim3 grid(a.max_chunks, a.Hq, batch);
+  if (a.sel == nullptr) {
+    a.batch = batch;
+    a.long_pages = dense_long_pages(a, head_dim);
+    a.split = 512u / a.Hq > 1u ? 512u / a.Hq : 1u;
+    // (every sequence of a few may end in a chunk of its own: still 512 in all)
+    if (batch > 1u && 4u * batch <= a.split) a.split -= batch;
+    a.long_split = 256u / a.Hkv > 1u ? 256u / a.Hkv : 1u;
+    a.split_rcp = rcp(a.split);
+    a.long_rcp = rcp(a.long_split);
+    const bool may_be_long = (uint64_t)a.max_pages * batch >= a.long_pages;
+    if (may_be_long || a.heads_per_item > 1u) G = a.Hq / a.Hkv;
+    const uint32_t split = may_be_long && a.long_split > a.split ? a.long_split : a.split;
+    // a sequence takes at most one item more than its share of the chunks
+    uint32_t items = batch > 1u ? split + batch : split < a.max_chunks ? split : a.max_chunks;
+    // (per-head workgroups of a group: whole sets of one per XCD)
+    if (G != a.Hq / a.Hkv)
+      while (items * a.Hkv % kXcds != 0u) ++items;
+    constexpr uint32_t kRows = 32768u;
+    grid = dim3(a.Hq / G, items < kRows ? items : kRows, (items + kRows - 1u) / kRows);
   }
-  const dim3 grid = dense ? dim3(heads, a.grid_chunks, batch) : dim3(a.grid_chunks, heads, batch);
   switch (head_dim) {
     case 64: return launch_d<64>(a, G, grid, s);
     case 128: return launch_d<128>(a, G, grid, s);

@@ -183,3 +183,20 @@ def test_graphed_decode_equals_forward(heads, kv_heads, single_launch):
         for mm in (eager, graphed):
             assert int(mm.iController.workspace[8:12].view(torch.int32).item()) == 0
             mm.quest_clear()
+
+
+@pytest.mark.parametrize("kv_heads", [32, 8])
+@pytest.mark.parametrize("n0", [1000, 2990, 5000])
+def test_graphed_decode_equals_forward_far_below_the_capacity(kv_heads, n0):
+    """32 heads in a cache for 32768 tokens: the dense layers' launches are
+    sized for it in the graph and for the sequence eagerly, with the same bits."""
+    _say(f"[shim-graph] heads=32 kv={kv_heads} {n0} tokens of 32768")
+    cfg = _cfg(4096, 32, kv_heads, layers=3)
+    eager, graphed = (_make(cfg, budget=512, max_len=32768) for _ in range(2))
+    g = torch.Generator(device=DEV).manual_seed(n0)
+    for step, n in enumerate([n0] + [1] * 5):
+        x = torch.randn(1, n, cfg.hidden_size, generator=g, device=DEV).half()
+        with torch.inference_mode():
+            want = eager(x)
+            got = graphed(x) if n > 1 else graphed.decode_graphed(x)
+        assert torch.equal(got, want), step
