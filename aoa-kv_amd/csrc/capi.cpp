@@ -962,6 +962,10 @@ size_t aoakv_prefill_workspace_size(uint32_t num_kv_pages, uint32_t kv_last_page
                                     uint32_t qo_len, uint32_t causal, uint32_t num_qo_heads,
                                     uint32_t head_dim, uint32_t page_size) {
   if (num_kv_pages == 0u || !aoakv::prefill_tuned_shape(head_dim, page_size)) return 0;
+  // (the call itself refuses these)
+  if (num_qo_heads == 0u || num_qo_heads > 256u || kv_last_page_len == 0u ||
+      kv_last_page_len > page_size)
+    return 0;
   const uint64_t L = (uint64_t)(num_kv_pages - 1u) * page_size + kv_last_page_len;
   if (qo_len == 0u || qo_len > L || L >= (1ull << 31)) return 0;
   return aoakv::prefill_plan((uint32_t)L, qo_len, causal ? 1u : 0u, num_qo_heads, head_dim)

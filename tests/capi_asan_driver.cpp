@@ -50,6 +50,18 @@ void sizes() {
   EXPECT(l >= d + 2u * 8u * 2048u * 4u);
   // the largest shapes the entry points accept do not overflow size_t
   EXPECT(aoakv_layer_workspace_size(65535, 64, 8, 256, 8192, 16384) > (size_t)1 << 32);
+  // a prefill's, of every shape the call itself takes and of some it refuses
+  for (uint32_t dim : {64u, 128u, 256u}) {
+    EXPECT(aoakv_prefill_workspace_size(1024, 16, 500, 1, 32, dim, 16) > 0);
+    EXPECT(aoakv_prefill_workspace_size(1024, 16, 500, 1, 0, dim, 16) == 0);
+    EXPECT(aoakv_prefill_workspace_size(1024, 16, 500, 1, 257, dim, 16) == 0);
+    EXPECT(aoakv_prefill_workspace_size(1024, 17, 500, 1, 32, dim, 16) == 0);
+    EXPECT(aoakv_prefill_workspace_size(1024, 0, 500, 1, 32, dim, 16) == 0);
+    for (uint32_t heads = 1; heads <= 256; heads += 5)
+      for (uint32_t qo : {1u, 129u, 4000u})
+        EXPECT(aoakv_prefill_workspace_size(70000, 16, qo, heads & 1u, heads, dim, 16) <=
+               (size_t)4 * 768 * 128 * (dim + 2) * 4);
+  }
 }
 
 void validation() {

@@ -201,6 +201,9 @@ def test_prefill_workspace_is_for_few_queries_over_many_keys():
     assert size(1024, 16, 500, 1, 32, 128, 16) > 0        # a chunk after 16k tokens
     assert size(1024, 16, 500, 1, 32, 128, 7) == 0        # not a shape of the split kernel
     assert size(0, 1, 1, 1, 32, 128, 16) == 0 and size(1, 16, 17, 1, 32, 128, 16) == 0
+    for D in (64, 128, 256):  # calls that are refused
+        assert size(1024, 16, 500, 1, 0, D, 16) == size(1024, 16, 500, 1, 257, D, 16) == 0
+        assert size(1024, 0, 500, 1, 32, D, 16) == size(1024, 17, 500, 1, 32, D, 16) == 0
     for D, slots in ((64, 768), (128, 512), (256, 256)):
         for pages in (64, 777, 4096, 65536):
             for qo in (1, 100, 129, 1000, 4000):
