@@ -1004,6 +1004,8 @@ int aoakv_prefill_with_workspace(const void* q, void* o, const void* kv_data,
           "prefill_with_paged_kv_cache: qo_len %u not in [1, %llu]", qo_len,
           (unsigned long long)L);
   REQUIRE(L < (1ull << 31), "prefill_with_paged_kv_cache: sequence too long");
+  REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16u == 0u,
+          "prefill_with_workspace: workspace not aligned to 16 bytes");
   aoakv::PrefillArgs a{};
   a.q = static_cast<const aoakv::f16*>(q);
   a.o = static_cast<aoakv::f16*>(o);

@@ -190,6 +190,16 @@ def test_noalloc_entry_point_rejects_without_gpu():
     assert rc == _lib.AOAKV_ERR_INVALID and b"error_bits" in lib.aoakv_last_error()
 
 
+def test_prefill_refuses_a_misaligned_workspace():
+    """The partials are stored 16 bytes at a time."""
+    from aoakv import _lib
+    lib = _lib.load()
+    n = lib.aoakv_prefill_workspace_size(1024, 16, 500, 1, 32, 128, 16)
+    rc = lib.aoakv_prefill_with_workspace(1 << 12, 2 << 12, 3 << 12, 4 << 12, 1024, 16, 500, 1, 32,
+                                          8, 128, 16, 1, (5 << 12) + 8, n, None)
+    assert rc == _lib.AOAKV_ERR_INVALID and b"16 bytes" in lib.aoakv_last_error()
+
+
 def test_prefill_workspace_is_for_few_queries_over_many_keys():
     """Calls whose query tiles fill the chip take no workspace; a split one's
     stays bounded (4 x 768 partials of 128 rows x 66 floats, 4 x 512 of 130 or
