@@ -86,9 +86,18 @@ const int32_t* i32_or_null(PyObject* o, const char* name) {
 }
 void* ptr(const Tensor& t) { return t.data_ptr(); }
 // the address of any tensor (the fused layer takes its page tables unchecked)
+void* any_ptr(PyObject* o, const char* name) {
+  if (!THPVariable_Check(o))
+    raise(PyExc_AttributeError, std::string(name) + " must be a torch.Tensor");
+  return THPVariable_Unpack(o).data_ptr();
+}
 const int32_t* table(PyObject* o) {
-  if (!THPVariable_Check(o)) raise(PyExc_AttributeError, "a page table must be a torch.Tensor");
-  return static_cast<const int32_t*>(THPVariable_Unpack(o).data_ptr());
+  return static_cast<const int32_t*>(any_ptr(o, "a page table"));
+}
+// v_log_norm: checked where the flags use it
+const void* log_norm_or_null(PyObject* o, uint32_t flags) {
+  if (flags & AOAKV_FLAG_VALUE_AWARE) return ptr(f16(o, "v_log_norm"));
+  return o == Py_None ? nullptr : any_ptr(o, "v_log_norm");
 }
 
 // An unsigned 32-bit argument: a Python int, as ctypes takes it.
@@ -97,6 +106,22 @@ uint32_t u32(PyObject* o) {
   const unsigned long v = PyLong_AsUnsignedLongMask(o);
   if (v == (unsigned long)-1 && PyErr_Occurred()) throw PyErr{};
   return (uint32_t)v;
+}
+// ... that is no more than a size: the whole number is compared
+uint32_t u32_at_most(PyObject* o, int64_t size, const char* msg) {
+  const uint32_t v = u32(o);
+  int big = 0;
+  const long long x = PyLong_AsLongLongAndOverflow(o, &big);
+  if (big != 0 || x < 0 || x > size) raise(PyExc_ValueError, msg);
+  return v;
+}
+// o == n, as Python compares them
+bool equals(PyObject* o, unsigned long n) {
+  PyObject* x = PyLong_FromUnsignedLong(n);
+  const int r = x == nullptr ? -1 : PyObject_RichCompareBool(o, x, Py_EQ);
+  Py_XDECREF(x);
+  if (r < 0) throw PyErr{};
+  return r != 0;
 }
 float f32(PyObject* o) {
   const double v = PyFloat_AsDouble(o);
@@ -111,8 +136,11 @@ struct Dims {
 Dims cache_dims(const Tensor& kv, PyObject* layout) {
   if (kv.dim() != 5 || kv.size(1) != 2)
     raise(PyExc_ValueError, "paged cache must be 5-d [pages, 2, ., ., D], got " + shape_str(kv));
+  if (!equals(layout, AOAKV_LAYOUT_NHD) && !equals(layout, AOAKV_LAYOUT_HND)) {
+    PyErr_Format(PyExc_ValueError, "unknown layout %S", layout);
+    throw PyErr{};
+  }
   const uint32_t l = u32(layout);
-  if (l > 1u) raise(PyExc_ValueError, "unknown layout " + std::to_string(l));
   const bool nhd = l == AOAKV_LAYOUT_NHD;
   return Dims{(uint32_t)kv.size(nhd ? 2 : 3), (uint32_t)kv.size(nhd ? 3 : 2),
               (uint32_t)kv.size(4), l};
@@ -167,9 +195,9 @@ void append_kv_cache_prefill(PyObject* const* a) {
     raise(PyExc_ValueError, "k/v must be [N, " + std::to_string(d.H) + ", " +
                                 std::to_string(d.D) + "], got " + shape_str(k) + " / " +
                                 shape_str(v));
-  const uint32_t pages = u32(a[4]), last = u32(a[5]);
-  if (THPVariable_Unpack(a[3]).numel() < (int64_t)pages)
-    raise(PyExc_ValueError, "kv_indices shorter than num_kv_pages");
+  const uint32_t pages = u32_at_most(a[4], THPVariable_Unpack(a[3]).numel(),
+                                     "kv_indices shorter than num_kv_pages"),
+                 last = u32(a[5]);
   void* s = stream();
   call("aoakv_append_kv_cache_prefill", [&] {
     return g_lib.append_kv_cache_prefill(ptr(k), ptr(v), (uint32_t)N, ptr(*c.kv), idx, pages,
@@ -194,9 +222,9 @@ void rope_append_kv_cache_prefill(PyObject* const* a) {
   if (q.dim() != 3 || q.size(0) != N || q.size(2) != d.D)
     raise(PyExc_ValueError, "q must be [" + std::to_string(N) + ", Hq, " + std::to_string(d.D) +
                                 "], got " + shape_str(q));
-  const uint32_t pages = u32(a[5]), last = u32(a[6]);
-  if (THPVariable_Unpack(a[4]).numel() < (int64_t)pages)
-    raise(PyExc_ValueError, "kv_indices shorter than num_kv_pages");
+  const uint32_t pages = u32_at_most(a[5], THPVariable_Unpack(a[4]).numel(),
+                                     "kv_indices shorter than num_kv_pages"),
+                 last = u32(a[6]);
   const float scale = f32(a[12]), theta = f32(a[13]);
   void* s = stream();
   call("aoakv_rope_append_kv_cache_prefill", [&] {
@@ -273,9 +301,7 @@ void estimate_attn_score(PyObject* const* a) {
                 *ip = i32(a[5], "kv_indptr"), *ix = i32(a[6], "kv_indices"),
                 *lpl = i32(a[7], "kv_last_page_len");
   const uint32_t max_pages = u32(a[9]), flags = u32(a[11]);
-  if (flags & AOAKV_FLAG_VALUE_AWARE) f16(a[8], "v_log_norm");
-  const void* log_norm =
-      a[8] == Py_None || !THPVariable_Check(a[8]) ? nullptr : ptr(THPVariable_Unpack(a[8]));
+  const void* log_norm = log_norm_or_null(a[8], flags);
   const Dims d = cache_dims(meta, a[10]);
   if (q.dim() != 3) raise(PyExc_ValueError, "q must be [B, Hq, D], got " + shape_str(q));
   if (q.size(2) != d.D || scores.dim() != 3 || scores.size(0) != q.size(0) ||
@@ -327,7 +353,7 @@ void decode_sparse_attn(PyObject* const* a) {
                 *lpl = i32(a[5], "kv_last_page_len"), *sel = i32_or_null(a[6], "sel_pages"),
                 *budgets = i32_or_null(a[12], "token_budgets");
   const Dims d = cache_dims(kv, a[11]);
-  if (d.H != u32(a[10])) raise(PyExc_ValueError, "num_kv_heads does not match kv_data");
+  if (!equals(a[10], d.H)) raise(PyExc_ValueError, "num_kv_heads does not match kv_data");
   if (q.dim() != 3) raise(PyExc_ValueError, "q must be [B, Hq, D], got " + shape_str(q));
   if (q.sizes() != o.sizes()) raise(PyExc_ValueError, "o must have q's shape");
   uint32_t sel_stride = 0u;
@@ -353,9 +379,7 @@ void sparse_decode_layer(PyObject* const* a) {
                &meta = f16(a[6], "metadata_data"), &scores = need(a[10], "scores", at::kFloat),
                &sel = need(a[11], "sel_pages", at::kInt), &ws = need(a[13], "workspace", at::kByte);
   const uint32_t flags = u32(a[16]);
-  if (flags & AOAKV_FLAG_VALUE_AWARE) f16(a[9], "v_log_norm");
-  const void* log_norm =
-      a[9] == Py_None || !THPVariable_Check(a[9]) ? nullptr : ptr(THPVariable_Unpack(a[9]));
+  const void* log_norm = log_norm_or_null(a[9], flags);
   const int32_t *budgets = i32_or_null(a[17], "token_budgets"), *ip = table(a[3]),
                 *ix = table(a[4]), *lpl = table(a[5]), *mip = table(a[7]), *mix = table(a[8]);
   const Dims d = cache_dims(kv, a[15]);

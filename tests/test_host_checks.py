@@ -71,3 +71,38 @@ def test_integers_layout_and_status():
     with pytest.raises(ops._lib.AoakvError, match="3 new tokens but the cache holds 2") as e:
         ops.append_kv_cache_prefill(k, k, cache, i(2), 1, 2, *rest, 1)
     assert e.value.code == ops._lib.AOAKV_ERR_INVALID
+
+
+@pytest.mark.gpu
+def test_integers_are_compared_whole():
+    """Arguments that are checked against a tensor's size (and the layout) are
+    not cut to 32 bits first, and the kv head count may be any number type;
+    a value statistic is a tensor whether the flags use it or not."""
+    import numpy as np
+    z = lambda *s: torch.zeros(s, dtype=H, device="cuda:0")
+    i = lambda *s: torch.zeros(s, dtype=I, device="cuda:0")
+    cache, k = z(2, 2, 4, 16, 128), z(3, 4, 128)
+    rest = (z(1, 2, 4, 16, 128), i(1), z(2, 4), z(2, 4, 128))
+    for pages in (2**32 + 1, 2**64 + 1, -1):
+        with pytest.raises(ValueError, match="kv_indices shorter"):
+            ops.append_kv_cache_prefill(k, k, cache, i(2), pages, 3, *rest, 1)
+        with pytest.raises(ValueError, match="kv_indices shorter"):
+            ops.rope_append_kv_cache_prefill(k.clone(), k.clone(), k, cache, i(2), pages, 3, *rest, 1)
+    for layout in (2**32 + 1, -1, 2**80):
+        with pytest.raises(ValueError, match=f"unknown layout {layout}"):
+            ops.append_kv_cache_prefill(k, k, cache, i(2), 1, 3, *rest, layout)
+    q, ip, last = z(1, 4, 128), torch.tensor([0, 1], **dict(dtype=I, device="cuda:0")), i(1) + 3
+    ws = ops.decode_workspace(1, 4, 4, 2, "cuda:0")
+    for heads in (np.int64(4), 4.0):
+        o = torch.full_like(q, float("nan"))
+        ops.decode_sparse_attn(q, o, cache, ip, i(2), last, None, 0, ws, 2, heads, 1)
+        assert torch.equal(o, torch.zeros_like(o))
+    for heads in (3, 2**32 + 4):
+        with pytest.raises(ValueError, match="num_kv_heads does not match"):
+            ops.decode_sparse_attn(q, o, cache, ip, i(2), last, None, 0, ws, 2, heads, 1)
+    scores = torch.zeros((1, 4, 2), device="cuda:0")
+    with pytest.raises(AttributeError):
+        ops.estimate_attn_score(q, scores, rest[0], ip, i(1), ip, i(2), last, "x", 2, 1, 0)
+    with pytest.raises(AttributeError):
+        ops.sparse_decode_layer(q, o, cache, ip, i(2), last, rest[0], ip, i(1), "x", scores,
+                                i(1, 4, 3), 32, ws, 2, 1, 0)
