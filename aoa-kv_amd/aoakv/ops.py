@@ -282,6 +282,9 @@ def estimate_topk(q, metadata_data, metadata_indptr, metadata_indices, kv_indptr
 def prefill_with_paged_kv_cache(q, kv_data, kv_indices, num_kv_pages: int, kv_last_page_len: int,
                                 layout: int, causal: bool = True, o=None):
     """Reference: quest/ops/csrc/batch_prefill.cu:27-117.  q [L, Hq, D] -> o;
-    the cache holds Hkv heads, Hq a multiple of Hkv (GQA)."""
+    the cache holds Hkv heads, Hq a multiple of Hkv (GQA).  A few queries over a
+    long context take scratch memory from torch's pool (at most 136 MB, see
+    aoakv_prefill_workspace_size), given back when the call returns; where the
+    pool has none the call runs without it, slower."""
     return _host.prefill_with_paged_kv_cache(q, o, kv_data, kv_indices, num_kv_pages,
                                              kv_last_page_len, layout, int(causal))

@@ -118,6 +118,27 @@ void validation() {
   EXPECT(rc == AOAKV_ERR_INVALID || launched_or_hip(rc));  // zero tokens: refused or a no-op
   rc = aoakv_apply_rope_in_place(fake(1), fake(2), 4, 0, 32, 32, 100, 1.0f, 1e4f, nullptr);
   EXPECT(rc != AOAKV_OK);
+  // a prompt's RoPE + append: null pointers, page length, positions, factors
+  auto rope_append = [&](void* q, uint32_t n, uint32_t heads, uint32_t pages, uint32_t last,
+                         float scale) {
+    return aoakv_rope_append_kv_cache_prefill(q, fake(2), fake(3), n, heads, fake(4),
+                                              fake<int32_t>(5), pages, last, fake(6),
+                                              fake<int32_t>(7), fake(8), fake(9), 8, 128, 16, 1,
+                                              scale, 1e4f, nullptr);
+  };
+  EXPECT(rope_append(nullptr, 100, 32, 7, 4, 1.0f) == AOAKV_ERR_INVALID);
+  EXPECT(rope_append(fake(1), 100, 0, 7, 4, 1.0f) == AOAKV_ERR_INVALID);
+  EXPECT(rope_append(fake(1), 100, 257, 7, 4, 1.0f) == AOAKV_ERR_INVALID);
+  EXPECT(rope_append(fake(1), 101, 32, 7, 4, 1.0f) == AOAKV_ERR_INVALID);
+  EXPECT(rope_append(fake(1), 100, 32, 7, 17, 1.0f) == AOAKV_ERR_INVALID);
+  EXPECT(rope_append(fake(1), 100, 32, 0, 4, 1.0f) == AOAKV_ERR_INVALID);
+  EXPECT(rope_append(fake(1), 100, 32, (1u << 20) + 1u, 1, 1.0f) == AOAKV_ERR_INVALID);
+  EXPECT(rope_append(fake(1), 100, 32, 7, 4, 0.0f) == AOAKV_ERR_INVALID);
+  // a prefill's workspace: alignment
+  rc = aoakv_prefill_with_workspace(fake(1), fake(2), fake(3), fake<int32_t>(4), 1024, 16, 500, 1,
+                                    32, 8, 128, 16, 1, static_cast<char*>(fake(5)) + 4, 1 << 30,
+                                    nullptr);
+  EXPECT(rc == AOAKV_ERR_INVALID && std::strstr(aoakv_last_error(), "16 bytes") != nullptr);
   // messages stay within the library's buffer
   rc = aoakv_workspace_init(nullptr, 0, nullptr);
   EXPECT(rc == AOAKV_ERR_INVALID && std::strlen(aoakv_last_error()) < 512);
@@ -184,6 +205,30 @@ void host_paths() {
     rc = aoakv_prefill_with_paged_kv_cache(fake(1), fake(2), fake(3), fake<int32_t>(4), 512, 16,
                                            8192, 1, 32, 8, 128, 16, layout, nullptr);
     EXPECT(launched_or_hip(rc));
+    for (uint32_t dim : {64u, 128u, 256u}) {  // split where the workspace holds it, else not
+      const size_t n = aoakv_prefill_workspace_size(1024, 16, 500, 1, 32, dim, 16);
+      for (size_t bytes : {n, n - 1u, (size_t)0})
+        EXPECT(launched_or_hip(aoakv_prefill_with_workspace(
+            fake(1), fake(2), fake(3), fake<int32_t>(4), 1024, 16, 500, 1, 32, 8, dim, 16, layout,
+            bytes != 0 ? fake(5) : nullptr, bytes, nullptr)));
+    }
+    // one pass, and two launches: shared memory, and another page size
+    for (uintptr_t v : {3u, 2u})
+      for (uint32_t page : {16u, 8u}) {
+        rc = aoakv_rope_append_kv_cache_prefill(fake(1), fake(2), fake(v), 100, 1, fake(400),
+                                                fake<int32_t>(5), 1600u / page, page, fake(6),
+                                                fake<int32_t>(7), fake(8), fake(9), 1, 128, page,
+                                                layout, 1.0f, 1e4f, nullptr);
+        EXPECT(launched_or_hip(rc));
+      }
+    // a batch's dense decode
+    for (uint32_t b : {2u, 64u, 65535u}) {
+      rc = aoakv_decode_sparse_attn(fake(1), fake(2), fake(3), fake<int32_t>(4),
+                                    fake<int32_t>(5), fake<int32_t>(6), nul, 0, 0, nul, fake(7),
+                                    aoakv_decode_workspace_size(b, Hq, Hkv, 128, 512), b, 512, Hq,
+                                    Hkv, 128, 16, layout, 0, nullptr);
+      EXPECT(launched_or_hip(rc));
+    }
   }
 }
 

@@ -236,3 +236,40 @@ def test_prefill_split_keys(L, Lq, Hq, Hkv, D, S, layout, causal):
         assert np.isfinite(got).all()
         assert np.abs(got[rows] - ref).max() <= 2e-3
     assert (o.float() - whole.float()).abs().max() <= 2e-3
+
+
+def test_prefill_without_room_for_its_workspace_runs_unsplit():
+    """torch's pool cannot give the partials' memory: the call runs without
+    them, with the bits of the call that is given no workspace."""
+    from aoakv import _lib, ops
+    Lq, L, Hq, Hkv = 300, 16000, 32, 8
+    P, last = L // S, S
+    g = torch.Generator(device=DEV).manual_seed(4)
+    rand = lambda *s: torch.randn(s, generator=g, device=DEV, dtype=torch.float16)
+    kv, q = rand(P, 2, Hkv, S, D), rand(Lq, Hq, D)
+    idx = torch.randperm(P, generator=g, device=DEV).int()
+    need = _lib.load().aoakv_prefill_workspace_size(P, last, Lq, 1, Hq, D, S)
+    assert need > 16 << 20
+    whole, o = torch.empty_like(q), torch.full_like(q, float("nan"))
+    _lib.call("aoakv_prefill_with_paged_kv_cache", q.data_ptr(), whole.data_ptr(), kv.data_ptr(),
+              idx.data_ptr(), P, last, Lq, 1, Hq, Hkv, D, S, HND,
+              torch.cuda.current_stream().cuda_stream)
+
+    def peak():
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        o.fill_(float("nan"))
+        ops.prefill_with_paged_kv_cache(q, kv, idx, P, last, HND, o=o)
+        return torch.cuda.max_memory_allocated() - before
+    assert peak() >= need
+    assert (o.float() - whole.float()).abs().max() <= 2e-3
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(DEV).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (4 << 20)) / total)
+    try:
+        assert peak() < need
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(o, whole)
