@@ -1,7 +1,8 @@
 """aoakv -- MI355X (gfx950) implementation of AOA-KV's decode hot path.
 
 Kernels live in libaoakv.so (hand-written HIP, C ABI in include/aoakv.h);
-this package binds them with ctypes and mirrors the reference's
+this package binds them with ctypes, and the append, decode and prefill
+calls through a C++ extension module (``_host``), and mirrors the reference's
 ``quest.utils`` interface in ``aoakv.utils``.  Importing the package loads
 the library and fails if it is missing: there is no fallback.
 """

@@ -67,8 +67,9 @@ def rope_append_kv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                    rope_scale: Optional[float] = None, rope_theta: Optional[float] = None):
     """apply_rope_in_place(q, k, seqlen - N) then append_kv(k, v) -- the
     reference's two calls at QuestAttention.py:98-111 -- in one launch (a
-    prompt at the shapes ops.rope_append_kv_cache_prefill names).  q and k are left rotated, as the reference leaves
-    them.  Call after begin_forward, like append_kv."""
+    prompt at the shapes ops.rope_append_kv_cache_prefill names).  q and k are
+    left rotated, as the reference leaves them.  Call after begin_forward, like
+    append_kv."""
     c = iController
     scale = 1.0 if rope_scale is None else rope_scale
     theta = 1e4 if rope_theta is None else rope_theta

@@ -88,7 +88,8 @@ uint32_t resident_layer_workgroups(uint32_t group, uint32_t heads_per_item, uint
   } while (0)
 
 // head_dim 64 / 128 / 256 (the reference's SWITCH_HEAD_DIM) and page sizes
-// 1..32; (128, 16) runs the tuned kernels, the rest generic.hip's
+// 1..32; (128, 16) runs the tuned kernels, the rest generic.hip's and
+// stream.hip's
 int check_shape(uint32_t head_dim, uint32_t page_size, uint32_t layout, uint32_t num_heads) {
   if (head_dim != 64u && head_dim != 128u && head_dim != 256u)
     return fail(AOAKV_ERR_UNSUPPORTED, "head_dim %u unsupported (64, 128, 256)", head_dim);
@@ -666,9 +667,10 @@ static int fill_decode(aoakv::DecodeArgs& a, Workspace& w, const void* q, void* 
                                         max_pages, page_size, flags);
   REQUIRE(!sel_pages || sel_stride >= min_sel_stride(flags), "decode_sparse_attn: sel_stride %u < %u",
           sel_stride, min_sel_stride(flags));
-  // both decode kernels split each head's pages over chunks of 8 merged
-  // through the workspace; the tuned merge holds at most decode_max_chunks
-  // of them, the generic one (chunk order, one workgroup) any number
+  // both decode kernels split each head's pages over chunks of 8 or more, merged
+  // through the workspace: decode.hip's merge holds at most decode_max_chunks
+  // of them (the limit of every call at the tuned shape), stream.hip's any
+  // number
   const bool tuned = aoakv::tuned_shape(head_dim, page_size);
   REQUIRE(!tuned || aoakv::decode_chunks(max_sel) <= aoakv::decode_max_chunks(),
           "decode_sparse_attn: %u pages per head exceed the %u the split-K merge holds", max_sel,
@@ -696,7 +698,7 @@ static int fill_decode(aoakv::DecodeArgs& a, Workspace& w, const void* q, void* 
   a.max_pages = max_pages;
   a.flags = flags & AOAKV_FLAG_QUEST_KERNEL;
   // grouped decode only where it changes anything (a group of 2 or more) and
-  // the tuned kernels run (the generic ones serve one query head each)
+  // the tuned kernels run (elsewhere a selection is one query head's at a time)
   a.heads_per_item =
       (flags & AOAKV_FLAG_GROUPED_DECODE) && tuned ? num_qo_heads / num_kv_heads : 1u;
   a.g = aoakv::make_geom(layout, num_kv_heads, page_size, head_dim);

@@ -162,8 +162,8 @@ __device__ inline f16 running_mean(f16 m, f16 v, uint32_t n) {
 // The sequential fp32 chain is carried lane to lane across the row: in step
 // s every lane adds its squares to the sum of the lane below (DPP row_shr:1, 0
 // below lane 0), so lane s holds the chain of lanes 0..s from step s on and
-// lane 15's is the row's after 16.  (The sum handed on by a shuffle through
-// the LDS unit in each step cost 0.8 us: a token's append 4.1 us, now 3.5.)
+// lane 15's is the row's after 16.  (With the sum handed on by a shuffle
+// through the LDS unit in each step a token's append took 4.1 us, now 3.5.)
 // Returns the fp16 log-norm in every lane of the row.
 __device__ inline f16 log_norm_row(const H8& vbar) {
   float sq[kVec];

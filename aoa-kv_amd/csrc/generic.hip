@@ -12,7 +12,8 @@
 //     (which takes any page size);
 //   * decode: stream.hip;
 //   * prefill: one lane group per query, keys in order with an online
-//     softmax, no MFMA (the tuned MFMA kernel covers (128, 16)).
+//     softmax, no MFMA (prefill.hip covers pages of 1, 2, 4, 8, 16 and
+//     32 tokens).
 // Arithmetic follows the tuned kernels where they define the reference's
 // rounding (fp16 filters, the fp32 page mean with one rounding, the fp16
 // running mean, the sequential fp32 norm of the log-norm).

@@ -256,8 +256,9 @@ uint32_t layer_stagger_ps(uint32_t est_chunks, uint32_t group, uint32_t heads); 
 uint32_t counter_stride();        // u32 words between per-head counters (one cache line each)
 uint32_t layer_self_blocks_per_cu(uint32_t group, uint32_t heads_per_item, uint32_t score_heads);  // per CU
 
-// stream.hip: dense decode (a.sel == nullptr, any shape), and the selected
-// pages of the shapes without tuned kernels
+// stream.hip: dense decode (a.sel == nullptr, any shape; a.heads_per_item > 1
+// reads K/V by GQA groups, with the same bits), and the selected pages of the
+// shapes without tuned kernels
 // self: the decode selects for itself, as launch_decode's (where stream_selects
 // says so)
 bool stream_selects(const DecodeArgs& a, uint32_t batch, uint32_t max_pages);

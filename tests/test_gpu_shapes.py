@@ -3,7 +3,7 @@ oracle, through the same C ABI: head_dim 64 / 128 / 256 (the reference's
 SWITCH_HEAD_DIM, decode_page.cuh:718-760, decode_attn.cuh:1159) and page
 sizes 1..32 (its page tests sweep 1, 3, 7, 16, 31, test_page.cu:600-683; its
 prefill takes 1, 8, 16, 32, prefill.cuh:1032-1036).  These shapes run the
-kernels of csrc/generic.hip.
+kernels of csrc/generic.hip and csrc/stream.hip.
 
 Bars as for the tuned shape: K/V storage, Kmax/Kmin, V̄ and log-norm
 bit-exact after a prefill and decode appends that cross pages; page scores
