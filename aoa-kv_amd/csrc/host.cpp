@@ -136,7 +136,10 @@ struct Dims {
 Dims cache_dims(const Tensor& kv, PyObject* layout) {
   if (kv.dim() != 5 || kv.size(1) != 2)
     raise(PyExc_ValueError, "paged cache must be 5-d [pages, 2, ., ., D], got " + shape_str(kv));
-  if (!equals(layout, AOAKV_LAYOUT_NHD) && !equals(layout, AOAKV_LAYOUT_HND)) {
+  int big = 0;
+  const long x = PyLong_Check(layout) ? PyLong_AsLongAndOverflow(layout, &big) : -1;
+  if (x != (long)AOAKV_LAYOUT_NHD && x != (long)AOAKV_LAYOUT_HND &&
+      !equals(layout, AOAKV_LAYOUT_NHD) && !equals(layout, AOAKV_LAYOUT_HND)) {
     PyErr_Format(PyExc_ValueError, "unknown layout %S", layout);
     throw PyErr{};
   }
