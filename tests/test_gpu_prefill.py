@@ -257,7 +257,6 @@ def test_prefill_without_room_for_its_workspace_runs_unsplit():
 
     def peak():
         torch.cuda.synchronize()
-        torch.cuda.empty_cache()
         torch.cuda.reset_peak_memory_stats()
         before = torch.cuda.memory_allocated()
         o.fill_(float("nan"))
@@ -268,7 +267,11 @@ def test_prefill_without_room_for_its_workspace_runs_unsplit():
     torch.cuda.empty_cache()
     total = torch.cuda.get_device_properties(DEV).total_memory
     torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (4 << 20)) / total)
+    filler = []  # what the pool still has in pieces of this size
     try:
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            while True:
+                filler.append(torch.empty(need, dtype=torch.uint8, device=DEV))
         assert peak() < need
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
